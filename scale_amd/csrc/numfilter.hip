@@ -3,7 +3,7 @@
 // Reference: ATMOS_DYN_numfilter_coef with ND_ORDER = 1 and ND_USE_RS,
 //   scalelib/src/atmos-rm/dynamics/scale_atmos_dyn_common.F90:385-985,
 //   calc_diff3 :1652-1800, coefficient tables filter_setup :92-319.
-// Blocks of 64 (i) x TJ (j) columns march k.  At each level the block
+// Blocks of 64 (i) x TJ (j) columns march a segment of levels.  At each level the block
 // evaluates the five differenced fields (DENS-REF_dens, w, u, v,
 // theta-REF_pott) once per tile cell (2-cell halo) into LDS for the x and y
 // differences; each column keeps the fields at k-2..k+2 in registers for the
@@ -52,9 +52,9 @@ __device__ __forceinline__ R phi_ref(R v, double ref) {
   else return R((double)v - ref);
 }
 
-// one tile (logical index lb of a grid ni_tiles tiles wide)
+// one tile (logical index lb of a grid ni_tiles tiles wide) over levels k0..k1
 template <int TJ, typename R>
-__device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigned lb, unsigned ni_tiles) {
+__device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigned lb, unsigned ni_tiles, int k0, int k1) {
   constexpr int TI = 64, CW = TI + 4, RW = TJ + 4, NT = TI * TJ;
   __shared__ R sD[2][RW + 1][CW + 1];  // DENS at k and k+1, one more cell east and north
   __shared__ R sP[5][RW][CW];          // the differenced fields at level k
@@ -117,7 +117,7 @@ __device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigne
   __syncthreads();
 
   // levels outside KS..KE are zero (KS-1 gets its DENS/RHOT z fluxes below)
-  if (own) {
+  if (own && k0 == KS) {
     for (int k = 0; k < d.KA; ++k) {
       if (k >= KS && k <= KE) continue;
       for (int q = 0; q < 15; ++q) out(q % 5, q / 5, k) = R(0);
@@ -128,13 +128,15 @@ __device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigne
   for (int f = 0; f < 5; ++f) for (int m = 0; m < 5; ++m) w[f][m] = R(0);
   if (own) {
     R ph[5];
-    for (int m = 3; m < 5; ++m) {  // shifted down once at the first level
-      phis(KS - 3 + m, ph);
+    for (int m = 1; m < 5; ++m) {  // shifted down once at the first level
+      const int k = k0 - 3 + m;
+      if (k < KS || k > KE) continue;
+      phis(k, ph);
       for (int f = 0; f < 5; ++f) w[f][m] = ph[f];
     }
   }
   int s0 = 0;
-  fillD(sD[0], KS);
+  fillD(sD[0], k0);
 
   // The global loads of level k, issued during the arithmetic of level k-1:
   // the raw fields of this thread's tile cells (the cells of the block's own
@@ -177,8 +179,8 @@ __device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigne
       oRD = a.REF_dens[q]; oRP = a.REF_pott[q];
     }
   };
-  if (KS <= KE) issue(KS);
-  for (int k = KS; k <= KE; ++k) {
+  issue(k0);
+  for (int k = k0; k <= k1; ++k) {
     const int s1 = s0 ^ 1;
 #pragma unroll
     for (int h = 0; h < NF; ++h) {
@@ -221,7 +223,7 @@ __device__ __forceinline__ void numfilter_tile_body(const NfArgsT<R>& a, unsigne
     }
     __syncthreads();
     // the next level's loads, in flight through this level's arithmetic
-    if (k < KE) issue(k + 1);
+    if (k < k1) issue(k + 1);
     if (own) {
       const int r = ty + 2, c = tx + 2;
       auto Dk = [&](int di, int dj) { return sD[s0][r + dj][c + di]; };
@@ -316,8 +318,10 @@ constexpr int nf_min_waves() { return (TJ == 8 && sizeof(R) == sizeof(float)) ? 
 
 template <int TJ, typename R>
 __global__ void __launch_bounds__(64 * TJ) __attribute__((amdgpu_waves_per_eu(nf_min_waves<TJ, R>())))
-numfilter_tile(NfArgsT<R> a, unsigned ni_tiles, unsigned nblocks) {
-  numfilter_tile_body<TJ, R>(a, xcd_block(blockIdx.x, nblocks), ni_tiles);
+numfilter_tile(NfArgsT<R> a, unsigned ni_tiles, unsigned ntile, unsigned nblocks, int L) {
+  const unsigned lb = xcd_block(blockIdx.x, nblocks);
+  const int k0 = a.d.KS + (int)(lb / ntile) * L;
+  numfilter_tile_body<TJ, R>(a, lb % ntile, ni_tiles, k0, min(a.d.KE, k0 + L - 1));
 }
 
 // the filters of many members in one launch (tables as hevi_tile_batch)
@@ -329,7 +333,7 @@ numfilter_tile_batch(const NfArgsT<R>* __restrict__ tab,
   for (unsigned t = blockIdx.x; t < total; t += gridDim.x) {
     const unsigned lt = xcd_block(t, total);
     const int lo = batch_member(first, nmem, lt);
-    numfilter_tile_body<TJ, R>(tab[lo], lt - first[lo], ni[lo]);
+    numfilter_tile_body<TJ, R>(tab[lo], lt - first[lo], ni[lo], tab[lo].d.KS, tab[lo].d.KE);
     __syncthreads();
   }
 }
@@ -369,13 +373,19 @@ static hipError_t numfilter_t(const Ctx& c, R* num_diff, const R* const st[5], c
     TJ = 4;
     if (ni * (unsigned)((jmax + 7) / 8) >= (unsigned)ncu) TJ = 8;
   }
-  const unsigned nj = (jmax + TJ - 1) / TJ;
-  const unsigned nb = ni * nj;
+  const unsigned nt = ni * (unsigned)((jmax + TJ - 1) / TJ);
+  // levels per block: a segment pays about three levels' work for its windows
+  // and its first ring level, and gives the device more blocks (a block's march
+  // waits on memory level by level: 329 -> 27 us at 40x40x80, 287 -> 69 at
+  // 128x128x64, 736 -> 637 at 320x320x96; one segment where the tiles fill the
+  // device, as at 512x512x128)
+  const int L = seg_levels(nt, d.KE - d.KS + 1, (unsigned)((TJ == 4 ? 2 : 1) + (TJ < 16 && sizeof(R) == sizeof(float) ? 1 : 0)) * (unsigned)ncu, 3.0);
+  const unsigned nb = nt * (unsigned)((d.KE - d.KS + L) / L);
   const size_t lds = 8 * (size_t)d.KA * sizeof(double);  // the z coefficient tables
   prof_start(c, "numfilter", s);
-  if (TJ == 16) hipLaunchKernelGGL((numfilter_tile<16, R>), dim3(nb), dim3(64, 16), lds, s, a, ni, nb);
-  else if (TJ == 8) hipLaunchKernelGGL((numfilter_tile<8, R>), dim3(nb), dim3(64, 8), lds, s, a, ni, nb);
-  else hipLaunchKernelGGL((numfilter_tile<4, R>), dim3(nb), dim3(64, 4), lds, s, a, ni, nb);
+  if (TJ == 16) hipLaunchKernelGGL((numfilter_tile<16, R>), dim3(nb), dim3(64, 16), lds, s, a, ni, nt, nb, L);
+  else if (TJ == 8) hipLaunchKernelGGL((numfilter_tile<8, R>), dim3(nb), dim3(64, 8), lds, s, a, ni, nt, nb, L);
+  else hipLaunchKernelGGL((numfilter_tile<4, R>), dim3(nb), dim3(64, 4), lds, s, a, ni, nt, nb, L);
   prof_stop(c, s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -53,6 +53,21 @@ struct Ctx {
   std::vector<double> hCDZ, hFDZ, hCDX, hFDX, hCDY, hFDY;
 };
 
+// Levels per segment of a tile march: ntile tiles, slots blocks resident at
+// once and pro levels' worth of work before a segment's first level.  The
+// march takes rounds x (levels + pro); the fewest segments among equals.
+inline int seg_levels(unsigned ntile, int kmax, unsigned slots, double pro) {
+  int best = kmax;
+  double cost = 1e30;
+  for (int ns = 1; ns <= (kmax + 3) / 4; ++ns) {
+    const int L = (kmax + ns - 1) / ns;
+    const unsigned nb = ntile * (unsigned)((kmax + L - 1) / L);
+    const double c = (double)((nb + slots - 1) / slots) * (L + pro);
+    if (c < cost) { cost = c; best = L; }
+  }
+  return best;
+}
+
 // one HEVI stage, all pointers in device layout; R is the storage type of the
 // prognostic, tendency, flux and num_diff arrays (float: mixed precision)
 template <typename R>

@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libscalehip.so")
-SOURCES = ["hevi.hip", "numfilter.hip", "tracer.hip", "tracer_tile.hip", "driver.hip", "adjoint.hip", "profile.hip",
+SOURCES = ["hevi.hip", "hevi_split.hip", "numfilter.hip", "tracer.hip", "tracer_tile.hip", "driver.hip", "adjoint.hip", "profile.hip",
            "metrics.hip", "capi.hip"]
 ARCH = os.environ.get("SCALE_HIP_ARCH", "gfx950")
 

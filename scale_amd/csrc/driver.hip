@@ -532,7 +532,7 @@ struct ShortBufs {
 template <typename R>
 static bool fused_rk4(const Ctx& c, bool batched) {
   const Model& M = *c.model;
-  return M.tinteg_short == 4 && !c.terrain && !M.heve && (sizeof(R) == sizeof(float) || batched || hevi_flat_tile(c));
+  return M.tinteg_short == 4 && !M.heve && (sizeof(R) == sizeof(float) || batched || hevi_fused_rk4(c));
 }
 
 template <typename R>

@@ -4,7 +4,7 @@
 //   scalelib/src/atmos-rm/dynamics/scale_atmos_dyn_tstep_short_fvm_hevi.F90:128-1089
 // with the flux stencils of scale_atmos_dyn_fvm_flux_{ud3,cd4}.F90.
 //
-// One kernel per stage.  Both kernels give each thread one column (i,j) and
+// One kernel per stage here.  Both kernels give each thread one column (i,j) and
 // march k upward through the explicit part of every point (pressure, mass and
 // theta fluxes, the explicit z fluxes, the tendencies Sr/St/Sw, the face value
 // PT, the complete MOMX/MOMY updates; HEVI.F90:346-657, 816-1047) and, one
@@ -15,69 +15,19 @@
 //   hevi_tile   flat terrain (GSQRT = 1, J13G = J23G = 0, MAPF = 1): blocks
 //               of 64 x 8 columns stage each level in LDS and evaluate every
 //               x and y face once;
-//   hevi_march  general metrics: neighbours come through the caches and each
+//   hevi_march  any metrics: neighbours come through the caches and each
 //               point evaluates the faces it needs.
+// General metrics and flat grids whose tiles leave CUs idle take the two
+// launches of hevi_split.hip instead; hevi_march remains for grids those do
+// not fit.
 #include <cstdlib>
 #include <vector>
 #include "common.h"
 #include "shp_internal.h"
 #include "batch.h"
+#include "hevi_args.h"
 
 namespace shp {
-
-// Arguments of a stage.  R is the type of the prognostic, tendency, flux and
-// num_diff arrays: double, or float for the mixed-precision path, which keeps
-// the reference state, the pressure terms (DPRES0, RT2P, REF_*) and the
-// vertical solve in double; the solve's coefficients e, f and the face
-// value PT pass from the upward to the downward sweep through scratch in R.
-template <typename R>
-struct HeviArgsT {
-  const Ctx* ctx;  // host side only
-  Dims d;
-  Grid1D g;
-  const double *GSQRT, *J13G, *J23G, *MAPF, *PHI;
-  double J33G;
-  // inputs (device layout)
-  const R *DENS0, *MOMZ0, *MOMX0, *MOMY0, *RHOT0;
-  const R *DENS, *MOMZ, *MOMX, *MOMY, *RHOT;
-  const R *DENS_t, *MOMZ_t, *MOMX_t, *MOMY_t, *RHOT_t;
-  const double *DPRES0, *RT2P, *CORIOLI;
-  const R* num_diff;
-  const double* wdamp_coef;
-  const R* DDIV;
-  const double *REF_dens, *REF_rhot;
-  double divdmp_coef, dtrk;
-  int has_coriolis;
-  // outputs
-  R *DENS_RK, *MOMZ_RK, *MOMX_RK, *MOMY_RK, *RHOT_RK, *mflx_hi, *tflx_hi;
-  // scratch (n3 each): in FP32 the Thomas coefficients are rounded to float
-  // between the sweeps (PT is a float value already), like the prognostics
-  R *PT, *e, *f;
-  // Sw between the two launches of the split terrain stage (FP64 only)
-  double* Sw = nullptr;
-  // optional records for the adjoint: St and the solved C
-  double *trSt = nullptr, *trCp = nullptr;
-  // mixed precision: DENS and RHOT (and their stage values) are stored as
-  // deviations from the level profiles offD(k), offR(k), kept in double
-  const double *offD = nullptr, *offR = nullptr;
-  // RK4 combination fused into the last stage (hevi_tile with CMB)
-  const R *c1[5], *c2[5], *c3[5];
-  const R *cm[3], *ct[3];
-  R* st[5];
-  R *mflx_av, *tflx_av;
-};
-using HeviArgs = HeviArgsT<double>;
-
-// RK4 combination (tinteg_short_rk4.F90:560-660): (2 r1 + 4 r2 + 2 r3 + r4 - 3 s0) / 6
-template <typename R>
-__device__ __forceinline__ R rk4c(R r1, R r2, R r3, R r4, R s0) {
-  return (r1 * R(2) + r2 * R(4) + r3 * R(2) + r4 - s0 * R(3)) / R(6);
-}
-// (f1 + 2 f2 + 2 f3 + f4) / 6
-template <typename R>
-__device__ __forceinline__ R rk4f(R f1, R f2, R f3, R f4) {
-  return (f1 + f2 * R(2) + f3 * R(2) + f4) / R(6);
-}
 
 template <int S, bool TERRAIN, bool DIVDMP>
 struct Ops {
@@ -434,12 +384,7 @@ __device__ __forceinline__ double momy_core(const Ops<S, TERRAIN, DIVDMP>& o, co
   return t;
 }
 
-// PART selects the sections evaluated (P_ALL for the whole point): the
-// continuity and theta fluxes with Sr and St (P_CT), the explicit part of
-// MOMZ with PT (P_W), MOMX (P_U) and MOMY (P_V); each section carries its
-// own z fluxes in zc.
-enum { P_CT = 1, P_W = 2, P_U = 4, P_V = 8, P_ALL = 15 };
-template <int S, bool TERRAIN, bool DIVDMP, int PART = P_ALL>
+template <int S, bool TERRAIN, bool DIVDMP>
 __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP>& o, const HeviArgs& a, int k, int i, int j,
                                                     ZCarry& zc) {
   const Dims& d = a.d;
@@ -451,7 +396,7 @@ __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP
   const auto& m = o.m;
 
   // ---- continuity (HEVI.F90:369-475) ----
-  if constexpr ((PART & P_CT) != 0) {
+  {
     const double mX = o.mflxX(k, i, j), mXm = o.mflxX(k, i - 1, j);
     const double mY = o.mflxY(k, i, j), mYm = o.mflxY(k, i, j - 1);
     r.mX = mX; r.mXm = mXm; r.mY = mY; r.mYm = mYm;
@@ -479,7 +424,7 @@ __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP
   }
 
   // ---- momentum z, explicit part (HEVI.F90:486-577) and PT (HEVI.F90:691) ----
-  if ((PART & P_W) != 0 && k <= d.KE - 1) {
+  if (k <= d.KE - 1) {
     const double qw = o.qZ_XYW(k, i, j);
     double sv = qw - zc.qW;
     zc.qW = qw;
@@ -500,7 +445,7 @@ __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP
   }
 
   // ---- momentum x (HEVI.F90:816-927), iee = min(IIE,IEH) = IE for periodic x ----
-  if constexpr ((PART & P_U) != 0) {
+  {
     double t = momx_core(o, a, k, i, j, zc);
     if constexpr (DIVDMP) {
       t = t + a.divdmp_coef / a.dtrk * (a.DDIV[IX(d, k, i + 1, j)] / m.mapf(i + 1, j, 1, I_XY) - a.DDIV[p] / m.mapf(i, j, 0, I_XY))
@@ -510,7 +455,7 @@ __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP
   }
 
   // ---- momentum y (HEVI.F90:936-1047) ----
-  if constexpr ((PART & P_V) != 0) {
+  {
     double t = momy_core(o, a, k, i, j, zc);
     if constexpr (DIVDMP) {
       t = t + a.divdmp_coef / a.dtrk * (a.DDIV[IX(d, k, i, j + 1)] / m.mapf(i, j + 1, 0, I_XY) - a.DDIV[p] / m.mapf(i, j, 0, I_XY))
@@ -524,11 +469,10 @@ __device__ __forceinline__ PointTend explicit_point(const Ops<S, TERRAIN, DIVDMP
 // The stores of one point, issued after all of its loads: the mass and
 // theta fluxes (with the extra faces i = IS-1, j = JS-1 and the zero z faces
 // KS-1 and KE, HEVI.F90:370-438, 596-622) and MOMX_RK/MOMY_RK.
-template <int PART = P_ALL>
 __device__ __forceinline__ void store_point(const HeviArgs& a, int k, int i, int j, const PointTend& r) {
   const Dims& d = a.d;
   const size_t p = IX(d, k, i, j);
-  if constexpr ((PART & P_CT) != 0) {
+  {
     double* mfZ = a.mflx_hi; double* mfX = a.mflx_hi + d.n3; double* mfY = a.mflx_hi + 2 * d.n3;
     double* tfZ = a.tflx_hi; double* tfX = a.tflx_hi + d.n3; double* tfY = a.tflx_hi + 2 * d.n3;
     mfX[p] = r.mX;
@@ -545,8 +489,8 @@ __device__ __forceinline__ void store_point(const HeviArgs& a, int k, int i, int
       if (k == d.KS) mfZ[p - 1 - d.pl] = 0.0;
     }
   }
-  if constexpr ((PART & P_U) != 0) a.MOMX_RK[p] = r.MX;
-  if constexpr ((PART & P_V) != 0) a.MOMY_RK[p] = r.MY;
+  a.MOMX_RK[p] = r.MX;
+  a.MOMY_RK[p] = r.MY;
 }
 
 // ---------------------------------------------------------------------------
@@ -672,270 +616,40 @@ __global__ void __launch_bounds__(256) hevi_march(HeviArgs a, unsigned ni_tiles,
   }
 }
 
-// ---------------------------------------------------------------------------
-// The same stage split in launches, the terrain stage's default
-// (hevi_march runs one thread per column: 16K columns at 128x128 are 256
-// waves, and the whole point needs 256 VGPRs).  hevi_expl: the explicit part
-// (the sections PART of it), one thread per segment of L levels of a column,
-// the carried z fluxes of the face below the segment computed afresh (the
-// carry of hevi_march at that face); it stores the mass and theta fluxes,
-// MOMX_RK/MOMY_RK, Sr/St (in DENS_RK/RHOT_RK), PT and Sw.  hevi_solve: one
-// thread per column, the tridiagonal system, its forward sweep and the back
-// substitution of hevi_march from those arrays.  The expressions and their
-// order are hevi_march's: the results are its bits.
-template <int S, bool TERRAIN, bool DIVDMP, int PART>
-__global__ void __launch_bounds__(256) hevi_expl(HeviArgs a, unsigned ni_tiles, unsigned ncols, unsigned nblocks, int L) {
-  const Dims& d = a.d;
-  Ops<S, TERRAIN, DIVDMP> o(a);
-  const unsigned lb = xcd_block(blockIdx.x, nblocks);
-  const unsigned col = lb % ncols, seg = lb / ncols;
-  const int i = d.IS + (int)((col % ni_tiles) * 64 + threadIdx.x);
-  const int j = d.JS + (int)((col / ni_tiles) * blockDim.y + threadIdx.y);
-  const int k0 = d.KS + (int)seg * L;
-  if (i > d.IE || j > d.JE || k0 > d.KE) return;
-  const int k1 = min(d.KE, k0 + L - 1);
-  constexpr bool PW = (PART & (P_CT | P_W)) != 0;  // the sections that read POTT around k
-  ZCarry zc;
-  if (k0 > d.KS) {
-    const int kb = k0 - 1;  // the face below the segment, as level kb of hevi_march leaves it
-    if constexpr ((PART & P_CT) != 0) {
-      double pw[4] = {o.POTT(kb - 1, i, j), o.POTT(kb, i, j), o.POTT(kb + 1, i, j), o.POTT(kb + 2, i, j)};
-      zc.mZ = o.mflxZf(kb, i, j);
-      zc.tZ = o.tflxZw(kb, i, j, zc.mZ, pw);
-    }
-    if constexpr ((PART & P_W) != 0) {
-      zc.qW = o.qZ_XYW(kb, i, j);
-      if constexpr (TERRAIN) { zc.qWJ13 = o.qJ_XYW(0, kb, i, j); zc.qWJ23 = o.qJ_XYW(1, kb, i, j); }
-    }
-    if constexpr ((PART & P_U) != 0) {
-      zc.qU = o.qZ_UV(0, kb, i, j);
-      if constexpr (TERRAIN) { zc.qUJ13 = o.qJ_UV(0, 0, kb, i, j); zc.qUJ23 = o.qJ_UV(0, 1, kb, i, j); }
-    }
-    if constexpr ((PART & P_V) != 0) {
-      zc.qV = o.qZ_UV(1, kb, i, j);
-      if constexpr (TERRAIN) { zc.qVJ13 = o.qJ_UV(1, 0, kb, i, j); zc.qVJ23 = o.qJ_UV(1, 1, kb, i, j); }
-    }
-  }
-  if constexpr (PW) { zc.pw[1] = o.POTT(k0 - 1, i, j); zc.pw[2] = o.POTT(k0, i, j); zc.pw[3] = o.POTT(k0 + 1, i, j); }
-  for (int k = k0; k <= k1; ++k) {
-    if constexpr (PW) {
-      zc.pw[0] = zc.pw[1]; zc.pw[1] = zc.pw[2]; zc.pw[2] = zc.pw[3];
-      zc.pw[3] = o.POTT(k + 2, i, j);
-    }
-    const PointTend t = explicit_point<S, TERRAIN, DIVDMP, PART>(o, a, k, i, j, zc);
-    const size_t q = IX(d, k, i, j);
-    store_point<PART>(a, k, i, j, t);
-    if constexpr ((PART & P_CT) != 0) {
-      a.DENS_RK[q] = t.Sr;
-      a.RHOT_RK[q] = t.St;
-      if (a.trSt) a.trSt[q] = t.St;
-    }
-    if constexpr ((PART & P_W) != 0) {
-      if (k <= d.KE - 1) { a.PT[q] = t.PT; a.Sw[q] = t.Sw; }
-    }
-  }
-}
-
-template <int S, bool TERRAIN, bool DIVDMP>
-__global__ void __launch_bounds__(256) hevi_solve(HeviArgs a, unsigned ni_tiles, unsigned nblocks) {
-  const Dims& d = a.d;
-  Ops<S, TERRAIN, DIVDMP> o(a);
-  const unsigned lb = xcd_block(blockIdx.x, nblocks);
-  const int i = d.IS + (int)((lb % ni_tiles) * 64 + threadIdx.x);
-  const int j = d.JS + (int)((lb / ni_tiles) * blockDim.y + threadIdx.y);
-  if (i > d.IE || j > d.JE) return;
-  const auto& m = o.m;
-  const double* CDZ = a.g.CDZ; const double* RCDZ = a.g.RCDZ; const double* RFDZ = a.g.RFDZ;
-  const double dtrk = a.dtrk, J33G = a.J33G;
-  const int KS = d.KS, KE = d.KE;
-  auto px = [&](int k) { return IX(d, k, i, j); };
-  auto dpres = [&](int k) { size_t q = px(k); return a.DPRES0[q] + a.RT2P[q] * (a.RHOT[q] - a.REF_rhot[q]); };
-  auto Af = [&](int k, double rt) { return dtrk * dtrk * J33G * RCDZ[k] * rt * J33G / m.gs(I_XYZ, px(k)); };
-  auto f2h = [&](int k, int pp) {
-    return CDZ[k + pp - 1] * m.gs(I_XYZ, px(k + pp - 1)) / (CDZ[k] * m.gs(I_XYZ, px(k)) + CDZ[k + 1] * m.gs(I_XYZ, px(k + 1)));
-  };
-  double* Sr_ = a.DENS_RK;
-  double* St_ = a.RHOT_RK;
-
-  // ---- upward: row k-1 of the system once level k is known; the loads of
-  //      level k+1 are issued before the work of level k ----
-  struct Up {
-    double rt, dp0, rh, rr, dn, rd, pt, st, sr, sw, mz;
-  };
-  auto up_load = [&](int k, Up& L) {
-    const size_t q = px(k);
-    L.rt = a.RT2P[q]; L.dp0 = a.DPRES0[q]; L.rh = a.RHOT[q]; L.rr = a.REF_rhot[q];
-    L.dn = a.DENS[q]; L.rd = a.REF_dens[q];
-    L.st = St_[q]; L.sr = Sr_[q];
-    const bool w = k <= KE - 1;
-    L.pt = w ? a.PT[q] : 0.0;
-    L.sw = w ? a.Sw[q] : 0.0;
-    L.mz = w ? a.MOMZ[q] : 0.0;
-  };
-  double rt0 = 0.0, dp0 = 0.0, st0 = 0.0, sr0 = 0.0, d0 = 0.0, rd0 = 0.0, A0 = 0.0, pt0 = 0.0, ptm = 0.0, sw0 = 0.0, mz0 = 0.0;
-  double e_prev = 0.0, f_prev = 0.0, C_last = 0.0;
-  Up cur{}, nxt{};
-  up_load(KS, cur);
-  for (int k = KS; k <= KE; ++k) {
-    if (k < KE) up_load(k + 1, nxt);
-    const double rt1 = cur.rt, dp1 = cur.dp0 + cur.rt * (cur.rh - cur.rr), d1 = cur.dn, rd1 = cur.rd, A1 = Af(k, rt1);
-    const double pt1 = cur.pt, st1 = cur.st, sr1 = cur.sr, sw1 = cur.sw;
-    double ek = 0.0, fk = 0.0;
-    if (k > KS) {
-      const int r = k - 1;
-      const size_t q = px(r);
-      const double gw = m.gs(I_XYW, q);
-      const double B = GRAV * (dtrk * dtrk) * J33G / (CDZ[r + 1] + CDZ[r]);
-      const double F1v = -(pt1 * RFDZ[r] * A1 + B) / gw;
-      const double F2v = 1.0 + (pt0 * RFDZ[r] * (A1 + A0)) / gw;
-      const double F3v = -(ptm * RFDZ[r] * A0 - B) / gw;
-      const double pg = -(dp1 + rt1 * dtrk * st1 - dp0 - rt0 * dtrk * st0) * RFDZ[r] * J33G / gw
-                      - GRAV * (f2h(r, 1) * (d1 - rd1 + sr1 * dtrk) + f2h(r, 2) * (d0 - rd0 + sr0 * dtrk));
-      const double Ck = mz0 + dtrk * (pg + sw0);
-      if (r == KS) {
-        const double rdenom = 1.0 / F2v;
-        ek = -F1v * rdenom;
-        fk = Ck * rdenom;
-      } else if (r < KE - 1) {
-        const double rdenom = 1.0 / (F2v + F3v * e_prev);
-        ek = -F1v * rdenom;
-        fk = (Ck - F3v * f_prev) * rdenom;
-      } else {
-        C_last = (Ck - F3v * f_prev) / (F2v + F3v * e_prev);
-      }
-      e_prev = ek; f_prev = fk;
-      ptm = pt0;
-      if (r < KE - 1) { a.e[q] = ek; a.f[q] = fk; }
-    }
-    rt0 = rt1; dp0 = dp1; st0 = st1; sr0 = sr1; d0 = d1; rd0 = rd1; A0 = A1; pt0 = pt1; sw0 = sw1; mz0 = cur.mz;
-    cur = nxt;
-  }
-
-  // ---- downward: back substitution and updates (HEVI.F90:728-790) ----
-  double* mfZ = a.mflx_hi; double* tfZ = a.tflx_hi;
-  const double M12 = m.mapf(i, j, 0, I_XY) * m.mapf(i, j, 1, I_XY);
-  double Cn = C_last;
-  double ptn = a.PT[px(KE - 1)];
-  {
-    const size_t q = px(KE);
-    double advcv = Cn * J33G * RCDZ[KE] / m.gs(I_XYZ, q);
-    a.DENS_RK[q] = a.DENS0[q] + dtrk * (advcv + Sr_[q]);
-    advcv = Cn * ptn * J33G * RCDZ[KE] / m.gs(I_XYZ, q);
-    a.RHOT_RK[q] = a.RHOT0[q] + dtrk * (advcv + St_[q]);
-    a.MOMZ_RK[q] = 0.0;
-  }
-  {
-    const size_t q = px(KE - 1);
-    mfZ[q] = mfZ[q] + J33G * Cn / (M12);
-    tfZ[q] = tfZ[q] + J33G * Cn * ptn / (M12);
-    a.MOMZ_RK[q] = a.MOMZ0[q] + (Cn - a.MOMZ[q]);
-    if (a.trCp) a.trCp[q] = Cn;
-  }
-  // the loads of level k-1 (and of level k's Sr/St/DENS0/RHOT0) are issued
-  // before the work of level k
-  struct Dn {
-    double e, f, pt, mz0, mz, mf, tf, d0, r0, sr, st;
-  };
-  auto dn_load = [&](int k, Dn& L) {
-    const size_t q = px(k), q1 = px(k + 1);
-    L.e = a.e[q]; L.f = a.f[q]; L.pt = a.PT[q]; L.mz0 = a.MOMZ0[q]; L.mz = a.MOMZ[q];
-    L.mf = mfZ[q]; L.tf = tfZ[q];
-    L.d0 = a.DENS0[q1]; L.r0 = a.RHOT0[q1]; L.sr = Sr_[q1]; L.st = St_[q1];
-  };
-  Dn dc{}, dn{};
-  if (KE - 2 >= KS) dn_load(KE - 2, dc);
-  for (int k = KE - 2; k >= KS; --k) {
-    if (k > KS) dn_load(k - 1, dn);
-    const size_t q = px(k), q1 = px(k + 1);
-    const double Ck = dc.e * Cn + dc.f;
-    const double ptk = dc.pt;
-    mfZ[q] = dc.mf + J33G * Ck / (M12);
-    tfZ[q] = dc.tf + J33G * Ck * ptk / (M12);
-    a.MOMZ_RK[q] = dc.mz0 + (Ck - dc.mz);
-    if (a.trCp) a.trCp[q] = Ck;
-    double advcv = -(Cn - Ck) * J33G * RCDZ[k + 1] / m.gs(I_XYZ, q1);
-    a.DENS_RK[q1] = dc.d0 + dtrk * (advcv + dc.sr);
-    advcv = -(Cn * ptn - Ck * ptk) * J33G * RCDZ[k + 1] / m.gs(I_XYZ, q1);
-    a.RHOT_RK[q1] = dc.r0 + dtrk * (advcv + dc.st);
-    Cn = Ck; ptn = ptk;
-    dc = dn;
-  }
-  {
-    const size_t q = px(KS);
-    double advcv = -Cn * J33G * RCDZ[KS] / m.gs(I_XYZ, q);
-    a.DENS_RK[q] = a.DENS0[q] + dtrk * (advcv + Sr_[q]);
-    advcv = -Cn * ptn * J33G * RCDZ[KS] / m.gs(I_XYZ, q);
-    a.RHOT_RK[q] = a.RHOT0[q] + dtrk * (advcv + St_[q]);
-    a.MOMZ_RK[px(KS - 1)] = 0.0;
-  }
-}
-
-// levels per segment of hevi_expl; SCALE_HIP_TERRAIN_SEG overrides the
-// default 8 (0: the single-launch hevi_march)
-static int terrain_seg_levels() {
+// The split stage (hevi_split.hip) runs the general-metrics stage and the flat
+// grids the tile kernel does not take; SCALE_HIP_TERRAIN_SEG=0 and grids it
+// does not fit (more than 512 levels) keep the single-launch march.
+static bool split_enabled(const Ctx& c) {
   const char* e = getenv("SCALE_HIP_TERRAIN_SEG");
-  return e ? atoi(e) : 8;
-}
-
-// the sections of hevi_expl per launch: SCALE_HIP_TERRAIN_PARTS lists the
-// section masks of the launches ("15": one launch; "3,12"; "1,2,4,8").  One
-// launch per section is the default: with the whole point in one launch a
-// thread needs 256 VGPRs (one wave per SIMD); per section 150-256, with two
-// to three waves for the momenta.  Measured at 128x128x64 / 512x512x128
-// (bell mountain, UD3): 1.07 / 25.4 ms per stage in one launch, 0.95 / 22.4
-// in two, 0.76 / 15.9 in four; hevi_march 2.92 / 27.6.
-static std::vector<int> terrain_parts() {
-  const char* e = getenv("SCALE_HIP_TERRAIN_PARTS");
-  std::vector<int> v;
-  for (const char* c = e ? e : "1,2,4,8"; *c;) {
-    char* end = nullptr;
-    const long m = strtol(c, &end, 10);
-    if (end == c) break;
-    v.push_back((int)m);
-    c = *end == ',' ? end + 1 : end;
-  }
-  return v;
+  return !(e && *e && atoi(e) <= 0) && hevi_split_fits(c.d);
 }
 
 template <int S, bool TERRAIN, bool DIVDMP>
-static void launch_split(const HeviArgs& a, hipStream_t s) {
+static hipError_t launch_march(const HeviArgs& a, hipStream_t s) {
   const Dims& d = a.d;
-  const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1, kmax = d.KE - d.KS + 1;
   constexpr unsigned TJ = 4;
-  const unsigned ni = (imax + 63) / 64, ncols = ni * ((jmax + TJ - 1) / TJ);
-  const int L = terrain_seg_levels();
-  if (L <= 0) {
-    hipLaunchKernelGGL((hevi_march<S, TERRAIN, DIVDMP>), dim3(ncols), dim3(64, TJ), 0, s, a, ni, ncols);
-    return;
-  }
-  const unsigned nseg = (unsigned)((kmax + L - 1) / L), nb = ncols * nseg;
-  const dim3 g(nb), b(64, TJ);
-  for (int part : terrain_parts()) {
-    switch (part) {
-      case P_ALL: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_ALL>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_CT | P_W: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_CT | P_W>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_U | P_V: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_U | P_V>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_CT: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_CT>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_W: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_W>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_U: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_U>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      case P_V: hipLaunchKernelGGL((hevi_expl<S, TERRAIN, DIVDMP, P_V>), g, b, 0, s, a, ni, ncols, nb, L); break;
-      default: break;
-    }
-  }
-  hipLaunchKernelGGL((hevi_solve<S, TERRAIN, DIVDMP>), dim3(ncols), dim3(64, TJ), 0, s, a, ni, ncols);
+  const unsigned ni = (unsigned)((d.IE - d.IS + 1 + 63) / 64), nb = ni * (unsigned)((d.JE - d.JS + 1 + (int)TJ - 1) / (int)TJ);
+  hipLaunchKernelGGL((hevi_march<S, TERRAIN, DIVDMP>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
+  return hipGetLastError();
 }
 
-// Flat grids whose 64 x 8 tiles do not give every CU a block (hevi_tile at
-// 128x128 is 32 blocks on 256 CUs) take the split launches instead; the RK4
-// combination then runs as its own kernel.  SCALE_HIP_FLAT_SPLIT=0 keeps the
-// tile kernel, =1 the split launches, whatever the grid.
+// The flat stage on the tile kernel, or split.  The tile kernel runs one block
+// a CU, so its time goes in rounds of ncu tiles: it takes grids whose tiles
+// fill at least 90 % of them.  RK4 short step, tile | split: 512x512x128 (two
+// full rounds) 20.5 | 21.5 ms, 512x512x64 10.2 | 10.3, 320x320x96 (0.78 of a
+// round) 7.0 | 6.8, 448x320x96 (1.09) 13.3 | 9.5, 128x128x64 (0.13) 3.6 |
+// 0.76.  SCALE_HIP_FLAT_SPLIT=0 keeps the tile kernel, =1 the split launches,
+// whatever the grid.
 bool hevi_flat_tile(const Ctx& c) {
   const char* e = getenv("SCALE_HIP_FLAT_SPLIT");
   if (e && *e) return atoi(e) == 0;
   const Dims& d = c.d;
-  const unsigned nt = (unsigned)((d.IE - d.IS + 1 + 63) / 64) * (unsigned)((d.JE - d.JS + 1 + 7) / 8);
-  return nt >= (unsigned)c.ncu;
+  const unsigned nt = (unsigned)((d.IE - d.IS + 1 + 63) / 64) * (unsigned)((d.JE - d.JS + 1 + 7) / 8), n = (unsigned)c.ncu;
+  return 10u * nt >= 9u * n * ((nt + n - 1) / n);
 }
+// the stage runs as the split launches
+static bool stage_split(const Ctx& c) { return (c.terrain || !hevi_flat_tile(c)) && split_enabled(c); }
+bool hevi_fused_rk4(const Ctx& c) { return stage_split(c) || (!c.terrain && hevi_flat_tile(c)); }
 
 // ---------------------------------------------------------------------------
 // HEVE: the fully explicit short step (ATMOS_DYN_Tstep_short_fvm_heve,
@@ -1805,27 +1519,18 @@ __global__ void __launch_bounds__(64 * TJ) hevi_tile_batch(const HeviArgsT<R>* _
 template <int S, bool TERRAIN, bool DIVDMP>
 static hipError_t launch_t(const HeviArgs& a, hipStream_t s, bool cmb) {
   const Dims& d = a.d;
-  const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1;
   const Ctx& c = *a.ctx;
-  const unsigned ni = (imax + 63) / 64;
-  prof_start(c, "hevi_stage", s);
+  if (stage_split(c)) return hevi_split(a, S, TERRAIN, DIVDMP, cmb, s);
   if constexpr (!TERRAIN) {
-    if (!cmb && !hevi_flat_tile(c)) {
-      launch_split<S, false, DIVDMP>(a, s);
-      prof_stop(c, s);
+    if (hevi_flat_tile(c)) {  // LDS tiles of 64 x 8 columns
+      constexpr int TJ = 8;
+      const unsigned ni = (unsigned)((d.IE - d.IS + 1 + 63) / 64), nb = ni * (unsigned)((d.JE - d.JS + 1 + TJ - 1) / TJ);
+      if (cmb) hipLaunchKernelGGL((hevi_tile<S, DIVDMP, TJ, double, true>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
+      else hipLaunchKernelGGL((hevi_tile<S, DIVDMP, TJ, double, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
       return hipGetLastError();
     }
-    // flat terrain: LDS tiles of 64 x 8 columns
-    constexpr int TJ = 8;
-    const unsigned nb = ni * ((jmax + TJ - 1) / TJ);
-    if (cmb) hipLaunchKernelGGL((hevi_tile<S, DIVDMP, TJ, double, true>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-    else hipLaunchKernelGGL((hevi_tile<S, DIVDMP, TJ, double, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-  } else {
-    if (cmb) { prof_stop(c, s); return hipErrorNotSupported; }
-    launch_split<S, true, DIVDMP>(a, s);
   }
-  prof_stop(c, s);
-  return hipGetLastError();
+  return cmb ? hipErrorNotSupported : launch_march<S, TERRAIN, DIVDMP>(a, s);
 }
 
 template <typename R>
@@ -1900,19 +1605,22 @@ hipError_t hevi_batch_launch(const BatchBuf& b, int bpc, int ncu, hipStream_t s)
   return b.cmb ? hevi_batch_launch_t<CD4, double, true>(b, bpc, ncu, s) : hevi_batch_launch_t<CD4, double, false>(b, bpc, ncu, s);
 }
 
+static hipError_t launch_any(const HeviArgs& a, bool div, bool cmb, hipStream_t s) {
+  const Ctx& c = *a.ctx;
+  if (c.scheme == UD3) {
+    if (c.terrain) return div ? launch_t<UD3, true, true>(a, s, cmb) : launch_t<UD3, true, false>(a, s, cmb);
+    return div ? launch_t<UD3, false, true>(a, s, cmb) : launch_t<UD3, false, false>(a, s, cmb);
+  }
+  if (c.terrain) return div ? launch_t<CD4, true, true>(a, s, cmb) : launch_t<CD4, true, false>(a, s, cmb);
+  return div ? launch_t<CD4, false, true>(a, s, cmb) : launch_t<CD4, false, false>(a, s, cmb);
+}
 hipError_t hevi_stage(const StageIO& io, hipStream_t s) {
   HeviArgs a;
   fill_args(a, io);
-  const Ctx& c = *io.ctx;
-  const bool div = io.divdmp_coef != 0.0;
-  const bool ter = c.terrain;
-  const bool cmb = io.combine != 0;
-  if (c.scheme == UD3) {
-    if (ter) return div ? launch_t<UD3, true, true>(a, s, cmb) : launch_t<UD3, true, false>(a, s, cmb);
-    return div ? launch_t<UD3, false, true>(a, s, cmb) : launch_t<UD3, false, false>(a, s, cmb);
-  }
-  if (ter) return div ? launch_t<CD4, true, true>(a, s, cmb) : launch_t<CD4, true, false>(a, s, cmb);
-  return div ? launch_t<CD4, false, true>(a, s, cmb) : launch_t<CD4, false, false>(a, s, cmb);
+  prof_start(*io.ctx, "hevi_stage", s);
+  const hipError_t e = launch_any(a, io.divdmp_coef != 0.0, io.combine != 0, s);
+  prof_stop(*io.ctx, s);
+  return e;
 }
 
 template <int S, bool TERRAIN, bool DIVDMP>
@@ -2143,32 +1851,13 @@ hipError_t heve_stage(const StageIO& io, hipStream_t s) {
 }
 
 // FP64 stage recording PT, St and the solved vertical momentum C for the
-// adjoint: hevi_tile on flat grids whose tiles fill the device, the split
-// launches (hevi_expl sections + hevi_solve) otherwise and with terrain
+// adjoint, by the kernels hevi_stage takes on this grid
 hipError_t hevi_stage_traced(const StageIO& io, double* PT, double* St, double* Cp, hipStream_t s) {
+  if (io.divdmp_coef != 0.0 || io.combine) return hipErrorNotSupported;
   HeviArgs a;
   fill_args(a, io);
-  const Ctx& c = *io.ctx;
-  if (io.divdmp_coef != 0.0 || io.combine) return hipErrorNotSupported;
   a.PT = PT; a.trSt = St; a.trCp = Cp;
-  const Dims& d = c.d;
-  const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1;
-  const unsigned ni = (imax + 63) / 64;
-  if (c.terrain) {
-    if (c.scheme == UD3) launch_split<UD3, true, false>(a, s);
-    else launch_split<CD4, true, false>(a, s);
-    return hipGetLastError();
-  }
-  if (!hevi_flat_tile(c)) {
-    if (c.scheme == UD3) launch_split<UD3, false, false>(a, s);
-    else launch_split<CD4, false, false>(a, s);
-    return hipGetLastError();
-  }
-  constexpr int TJ = 8;
-  const unsigned nb = ni * ((jmax + TJ - 1) / TJ);
-  if (c.scheme == UD3) hipLaunchKernelGGL((hevi_tile<UD3, false, TJ, double, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-  else hipLaunchKernelGGL((hevi_tile<CD4, false, TJ, double, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-  return hipGetLastError();
+  return launch_any(a, false, false, s);
 }
 
 hipError_t hevi_stage(const StageIOT<float>& io, hipStream_t s) {

@@ -141,6 +141,8 @@ hipError_t hevi_batch_launch(const BatchBuf& b, int blocks_per_cu, int ncu, hipS
 // the flat FP64 stage on LDS tiles (false: the split launches, for grids
 // too small to give every CU a tile)
 bool hevi_flat_tile(const Ctx& c);
+// the FP64 stage takes the fused RK4 combination (tile kernel or split launches)
+bool hevi_fused_rk4(const Ctx& c);
 // the numerical filter of every member (then each member's halo fill)
 template <typename R>
 struct NfIn {

@@ -1,0 +1,62 @@
+"""The split FP64 stage (hevi_etile + hevi_columns) at the sizes where it can go
+wrong: tile, segment and column-block edges, remainders, the fewest levels, and
+level counts on both sides of every column-block width, bit for bit against the
+oracle; the RK4 combination fused into both kernels."""
+import numpy as np
+import pytest
+
+import helpers as H
+import pyoracle as po
+from scale_amd import inputs
+from test_gpu_parity import OUTS, hip, oracle_stage, run_stage_gpu  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# (kmax, imax, jmax): the fewest levels and columns; one column past a 32-column tile; one row past a tile; 256 rows
+# of columns and more (32 columns a block up to 64 levels, 16 beyond), few columns and 256 | 257 levels (8 a block);
+# 129 tiles of 64 columns (the wide tile)
+SIZES = [(4, 2, 2), (5, 33, 9), (9, 31, 17), (6, 33, 130), (65, 18, 130), (129, 9, 4), (257, 6, 3), (5, 65, 520)]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("terrain", [False, True], ids=["flat", "terrain"])
+@pytest.mark.parametrize("scheme", [3, 4], ids=["UD3", "CD4"])
+def test_stage_sizes(hip, size, terrain, scheme, monkeypatch):  # noqa: F811
+    monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", "1")
+    print(f"[split stage] {size} terrain={terrain} scheme={scheme}", flush=True)
+    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=31, dz=80.0)
+    inp = H.stage_inputs(case, seed=29, coriolis=True)
+    inp["wdamp_coef"] = np.linspace(0.0, 0.01, case.grid.KA)
+    inp["divdmp_coef"] = 0.1 if size[2] % 2 else 0.0
+    inp["DDIV"] = np.asfortranarray(np.random.Generator(np.random.PCG64(4)).standard_normal(case.grid.shape) * 1e-3)
+    metric = H.terrain_metrics(case) if terrain else None
+    ref = oracle_stage(case, inp, 0.5, metric, scheme)
+    got = run_stage_gpu(hip, case, inp, 0.5, metric, scheme)
+    for k in OUTS:
+        H.compare(ref[k], got[k], k)
+
+
+@pytest.mark.parametrize("size", [(4, 2, 2), (9, 65, 9), (33, 30, 7), (70, 33, 6)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("terrain", [False, True], ids=["flat", "terrain"])
+def test_fused_combination(hip, size, terrain, monkeypatch):  # noqa: F811
+    """Three large steps through the combining fourth stage, within 1e-12 of
+    each field's scale (pow() in the preparation)."""
+    monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", "1")
+    print(f"[split stage] model {size} terrain={terrain}", flush=True)
+    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=37, dz=100.0)
+    zs = inputs.bell_topography(case.grid, height=60.0, half_width=1500.0) if terrain else None
+    ocase = case
+    if terrain:
+        ocase = inputs.Case(**{**case.__dict__, "metric": {**case.metric, **po.terrain_metrics(case.grid, zs, case.fz, case.metric)}})
+    m = po.Model(ocase)
+    m.step(3)
+    g = case.grid
+    sl = (slice(g.KS, g.KE + 1), slice(g.IS, g.IE + 1), slice(g.JS, g.JE + 1))
+    with hip.model_from_case(case, zsfc=zs) as ctx:
+        ctx.model_large_step(3)
+        for k in hip.STATE:
+            got, ref = ctx.model_get(k), m.state[k]
+            assert np.abs(got - ref).max() <= 1e-12 * max(np.abs(ref).max(), 1.0), k  # ghost levels and halos too
+        for k in ("mflx_hi", "tflx_hi"):
+            got, ref = ctx.model_get(k)[sl], getattr(m, k)[sl]
+            assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max(), k

@@ -554,6 +554,8 @@ static StageIOT<R> short_stage_io(Ctx& c, double dts, const ShortBufs<R>& B, int
     io.s[v] = r == 0 ? B.st[v] : Rk(r - 1, v);
     io.t[v] = B.t[v];
   }
+  // (an ensemble's argument tables outlive a later model_set of a tendency)
+  io.t_zero = !batched && M.tend_zero;
   io.mflx_hi = B.mfR[r];
   io.tflx_hi = B.tfR[r];
   io.DPRES0 = M.DPRES0; io.RT2P = M.RT2P; io.CORIOLI = M.CORIOLI; io.num_diff = num_diff;

@@ -1053,7 +1053,8 @@ __device__ __forceinline__ void hevi_tile_body(const HeviArgsT<R>& a, unsigned l
     if (own || PIPE) {
       o_nZD = nd(I_DENS, ZDIR, gk); o_nZT = nd(I_RHOT, ZDIR, gk); o_nZW = nd(I_MOMZ, ZDIR, gk + d.pl);
       o_nZX = nd(I_MOMX, ZDIR, gk); o_nZY = nd(I_MOMY, ZDIR, gk);
-      o_Dt = a.DENS_t[gk]; o_Rt = a.RHOT_t[gk]; o_Wt = a.MOMZ_t[gk]; o_Xt = a.MOMX_t[gk]; o_Yt = a.MOMY_t[gk];
+      const size_t gt = gk & a.tmask;
+      o_Dt = a.DENS_t[gt]; o_Rt = a.RHOT_t[gt]; o_Wt = a.MOMZ_t[gt]; o_Xt = a.MOMX_t[gt]; o_Yt = a.MOMY_t[gt];
       o_X0 = a.MOMX0[gk]; o_Y0 = a.MOMY0[gk]; o_RT = a.RT2P[gk]; o_RD = a.REF_dens[gk];
       if constexpr (PIPE) {
         const R z0 = a.MOMZ0[gk];
@@ -1543,6 +1544,7 @@ static void fill_args(HeviArgsT<R>& a, const StageIOT<R>& io) {
   a.DENS0 = io.s0[0]; a.MOMZ0 = io.s0[1]; a.MOMX0 = io.s0[2]; a.MOMY0 = io.s0[3]; a.RHOT0 = io.s0[4];
   a.DENS = io.s[0]; a.MOMZ = io.s[1]; a.MOMX = io.s[2]; a.MOMY = io.s[3]; a.RHOT = io.s[4];
   a.DENS_t = io.t[0]; a.MOMZ_t = io.t[1]; a.MOMX_t = io.t[2]; a.MOMY_t = io.t[3]; a.RHOT_t = io.t[4];
+  a.tmask = io.t_zero ? 0 : ~(size_t)0;
   a.DPRES0 = io.DPRES0; a.RT2P = io.RT2P; a.CORIOLI = io.CORIOLI; a.num_diff = io.num_diff;
   a.wdamp_coef = io.wdamp_coef; a.DDIV = io.DDIV; a.REF_dens = io.REF_dens; a.REF_rhot = io.REF_rhot;
   a.divdmp_coef = io.divdmp_coef; a.dtrk = io.dtrk; a.has_coriolis = io.has_coriolis;

@@ -23,6 +23,9 @@ struct HeviArgsT {
   const R *DENS0, *MOMZ0, *MOMX0, *MOMY0, *RHOT0;
   const R *DENS, *MOMZ, *MOMX, *MOMY, *RHOT;
   const R *DENS_t, *MOMZ_t, *MOMX_t, *MOMY_t, *RHOT_t;
+  // elements the tendencies are read at: index & tmask (0 where all five are
+  // zero: every lane then reads element 0, one cached line instead of 5 arrays)
+  size_t tmask = ~(size_t)0;
   const double *DPRES0, *RT2P, *CORIOLI;
   const R* num_diff;
   const double* wdamp_coef;

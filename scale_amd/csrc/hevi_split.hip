@@ -290,18 +290,19 @@ __global__ void __launch_bounds__(TI * TJ, 2) hevi_etile(HeviArgs a, unsigned ni
     double o_RT = 0, o_RD = 0, o_P0 = 0, o_RR = 0, o_R = 0;
     const double wdc = a.wdamp_coef[k];
     if (own) {
+      const unsigned gt = g & (unsigned)a.tmask;
       if constexpr (PT_) { o_nZD = nd(I_DENS, ZDIR, g); o_nZT = nd(I_RHOT, ZDIR, g); o_nZW = nd(I_MOMZ, ZDIR, g + pl); }
       if constexpr (PM_) { o_nZX = nd(I_MOMX, ZDIR, g); o_nZY = nd(I_MOMY, ZDIR, g); }
       if (live) {
         if constexpr (PT_) {
-          o_Dt = ld(a.DENS_t, g); o_Rt = ld(a.RHOT_t, g); o_Wt = ld(a.MOMZ_t, g);
+          o_Dt = ld(a.DENS_t, gt); o_Rt = ld(a.RHOT_t, gt); o_Wt = ld(a.MOMZ_t, gt);
           o_RT = ld(a.RT2P, g); o_RD = ld(a.REF_dens, g);
           if constexpr (!PM_) { o_P0 = ld(a.DPRES0, g); o_RR = ld(a.REF_rhot, g); o_R = ld(a.RHOT, g); }
           if (TERRAIN || wdc != 0.0) o_Z0 = ld(a.MOMZ0, g);
           if (i == d.IS && k <= KE - 1) o_nDw = nd(I_DENS, ZDIR, g - 8);
         }
         if constexpr (PM_) {
-          o_Xt = ld(a.MOMX_t, g); o_Yt = ld(a.MOMY_t, g);
+          o_Xt = ld(a.MOMX_t, gt); o_Yt = ld(a.MOMY_t, gt);
           o_X0 = ld(a.MOMX0, g); o_Y0 = ld(a.MOMY0, g);
           if constexpr (CMB) {
 #pragma unroll

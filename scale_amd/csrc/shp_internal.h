@@ -78,6 +78,7 @@ struct StageIOT {
   const R* s0[5];           // DENS0..RHOT0
   const R* s[5];            // DENS..RHOT
   const R* t[5];            // DENS_t..RHOT_t
+  int t_zero = 0;           // all five are zero everywhere
   const double *DPRES0, *RT2P, *CORIOLI;
   const R* num_diff;
   const double* wdamp_coef;

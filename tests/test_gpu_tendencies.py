@@ -1,0 +1,39 @@
+"""Tendencies given to a model after steps without any, against the oracle."""
+import numpy as np
+import pytest
+
+import helpers as H
+import pyoracle as po
+from scale_amd import inputs
+from test_gpu_parity import hip  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("split", ["0", "1"], ids=["tile", "split"])
+def test_tendencies_given_later(hip, split, monkeypatch):  # noqa: F811
+    """Two steps without tendencies, which the stage then does not read, then
+    two with them: 1e-12 of the oracle."""
+    monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", split)
+    case = H.small_case(kmax=10, imax=9, jmax=6, seed=43)
+    g = case.grid
+    rng = np.random.Generator(np.random.PCG64(8))
+    tp = {}
+    for v in hip.STATE:
+        a = g.zeros()
+        a[:, g.IS:g.IE + 1, g.JS:g.JE + 1] = 1e-3 * rng.standard_normal((g.KA, g.imax, g.jmax))
+        tp[v + "_tp"] = inputs.halo_fill(g, a)
+    m = po.Model(case)
+    m.step(2)
+    later = po.Model(inputs.Case(**{**case.__dict__, "zero_tend": {**case.zero_tend, **tp}}))
+    later.state = {k: np.array(v, order="F", copy=True) for k, v in m.state.items()}
+    later.qtrc = np.array(m.qtrc, order="F", copy=True)
+    later.step(2)
+    with hip.model_from_case(case) as ctx:
+        ctx.model_large_step(2)
+        for k, v in tp.items():
+            ctx.model_set(k, v)
+        ctx.model_large_step(2)
+        for k in hip.STATE:
+            ref = later.state[k]
+            assert np.abs(ctx.model_get(k) - ref).max() <= 1e-12 * np.abs(ref).max(), k

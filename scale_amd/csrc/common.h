@@ -63,6 +63,17 @@ __host__ __device__ inline size_t IX(const Dims& d, int k, int i, int j) {
   return (size_t)i + (size_t)d.IA * (size_t)j + d.pl * (size_t)k;
 }
 
+// Element of a field at a byte offset: a uniform base in scalar registers and
+// a 32-bit vector offset, one VGPR per point instead of a 64-bit address per
+// load.  A field is smaller than 4 GiB (TILE_MAX_N3 elements).
+constexpr size_t TILE_MAX_N3 = (size_t)1 << 29;
+__device__ __forceinline__ double ld(const double* b, unsigned o) {
+  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(b) + o);
+}
+__device__ __forceinline__ void sto(double* b, unsigned o, double v) {
+  *reinterpret_cast<double*>(reinterpret_cast<char*>(b) + o) = v;
+}
+
 // Fortran sign(a,b)
 __device__ __forceinline__ double fsign(double a, double b) { return __builtin_copysign(__builtin_fabs(a), b); }
 __device__ __forceinline__ float fsign(float a, float b) { return __builtin_copysignf(__builtin_fabsf(a), b); }

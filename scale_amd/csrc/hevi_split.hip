@@ -20,15 +20,6 @@
 
 namespace shp {
 
-// Element of a field at a byte offset: a uniform base in scalar registers and
-// a 32-bit vector offset, one VGPR per point instead of a 64-bit address per
-// load (hevi_split_fits: a field is smaller than 4 GiB).
-__device__ __forceinline__ double ld(const double* b, unsigned o) {
-  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(b) + o);
-}
-__device__ __forceinline__ void sto(double* b, unsigned o, double v) {
-  *reinterpret_cast<double*>(reinterpret_cast<char*>(b) + o) = v;
-}
 // the metric accessors of Met on byte offsets
 template <bool TERRAIN>
 struct MetO {
@@ -877,7 +868,7 @@ __global__ void __launch_bounds__(1024) hevi_columns(HeviArgs a, unsigned ni, un
 }
 
 // the tridiagonal rows of 8 columns fit in LDS, a field's byte offsets in 32 bits
-bool hevi_split_fits(const Dims& d) { return d.KE - d.KS + 1 <= SOLVE_KMAX && d.n3 < ((size_t)1 << 29); }
+bool hevi_split_fits(const Dims& d) { return d.KE - d.KS + 1 <= SOLVE_KMAX && d.n3 < TILE_MAX_N3; }
 
 // Tiles of TI x 8 columns.  64 columns re-read the smaller halo (1.59 cells per
 // column against 1.69) and are the faster from about half a tile per CU on; 32

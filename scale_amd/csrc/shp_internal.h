@@ -120,6 +120,9 @@ struct TracerIO {
   const double *QTRC, *QTRC0, *RHOQ_t, *DENS0, *DENS, *mflx_hi, *num_diff;
   double dtl;
   int flag_fct, flag_along;
+  // stage without FCT on DENS0 + (DENS - DENS0) / 3 (1) or * 0.5 (2), the RK3
+  // stages' densities (tinteg_tracer_rk3.F90:140-147, 168-175); 0: on DENS
+  int dens_mode = 0;
 };
 
 // ---- ensembles: one launch over the tiles of many members' grids ----
@@ -200,12 +203,10 @@ hipError_t numfilter(const Ctx& c, double* num_diff, const double* const st[5], 
 hipError_t numfilter(const Ctx& c, float* num_diff, const float* const st[5], const double* REF_dens,
                      const double* REF_pott, hipStream_t s, const double* offD, const double* offR);
 hipError_t tracer_stage(const Ctx& c, const TracerIO& io, hipStream_t s);
-// the LDS-tiled tracer stage (flat terrain; UD3, CD4, UD3KOREN1993, UD1, CD2)
-// with R+/R- in the given fields; tracer_stage uses it where it applies
+// the LDS-tiled tracer stage (UD3, CD4, UD3KOREN1993, UD1, CD2), with FCT (R+/R-
+// in the given fields) or without; tracer_stage uses it where it applies
 bool tracer_tile_supported(const Ctx& c);
 hipError_t tracer_stage_tile(const Ctx& c, const TracerIO& io, double* rjpls, double* rjmns, hipStream_t s);
-// the stage without FCT on the same tiles (flat, two-cell schemes)
-hipError_t tracer_nofct_tile(const Ctx& c, const TracerIO& io, hipStream_t s);
 // the same on caller-supplied device metrics (GSQRT(..,7), MAPF(IA,JA,2),
 // RCDZ/RCDX/RCDY) and work arrays (3 n3 doubles: phi_lo, R+, R-)
 hipError_t tracer_stage_ext(const Ctx& c, const TracerIO& io, const double* GSQRT, const double* MAPF_XY,

@@ -33,6 +33,7 @@ struct TrArgs {
   double dtl;
   double* QTRCo;
   double *phi_lo, *rjpls, *rjmns;  // scratch
+  int dens_mode = 0;               // stage without FCT: its density (TracerIO)
 };
 
 template <int S, bool TERRAIN>
@@ -55,6 +56,10 @@ struct TrOps {
   // which gives the same sums as zeros loaded from memory
   __device__ __forceinline__ double ndv(size_t q) const { return a.nd ? a.nd[q] : 0.0; }
   __device__ __forceinline__ double rqv(size_t q) const { return a.RHOQ_t ? a.RHOQ_t[q] : 0.0; }
+  __device__ __forceinline__ double dens(size_t p) const {
+    const double d0 = a.DENS0[p], d1 = a.DENS[p];
+    return a.dens_mode == 1 ? d0 + (d1 - d0) / 3.0 : a.dens_mode == 2 ? d0 + (d1 - d0) * 0.5 : d1;
+  }
   __device__ __forceinline__ double mZ(size_t p) const { return a.mflx[p]; }
   __device__ __forceinline__ double mX(size_t p) const { return a.mflx[p + d.n3]; }
   __device__ __forceinline__ double mY(size_t p) const { return a.mflx[p + 2 * d.n3]; }
@@ -153,7 +158,7 @@ __device__ __forceinline__ void tracer_nofct_body(const TrArgs& a, unsigned lb, 
                              + (o.hY(k, i, j) - o.hY(k, i, j - 1)) * a.RCDY[j])
                            * o.m1(i, j) * o.m2(i, j) / o.gs(I_XYZ, p)
                            + o.rqv(p)))
-             / a.DENS[p];
+             / o.dens(p);
 }
 template <int S, bool TERRAIN>
 __global__ void __launch_bounds__(256) tracer_nofct(TrArgs a, unsigned ni_tiles, unsigned nk_tiles, unsigned nblocks) {
@@ -462,10 +467,9 @@ hipError_t tracer_stage_ext(const Ctx& c, const TracerIO& io, const double* GSQR
 }
 
 hipError_t tracer_stage(const Ctx& c, const TracerIO& io, hipStream_t s) {
-  // flat terrain with a two-cell scheme and a grid with blocks enough: the
-  // LDS-tiled kernels (tracer_tile.hip), with FCT or without
-  if (io.flag_fct && c.tracer_tile && tracer_tile_supported(c)) return tracer_stage_tile(c, io, c.scr[1], c.scr[2], s);
-  if (!io.flag_fct && c.tracer_tile && tracer_tile_supported(c)) return tracer_nofct_tile(c, io, s);
+  // a two-cell scheme and a grid with blocks enough: the LDS-tiled kernels
+  // (tracer_tile.hip), with FCT or without
+  if (c.tracer_tile && tracer_tile_supported(c)) return tracer_stage_tile(c, io, c.scr[1], c.scr[2], s);
   TrArgs a;
   a.d = c.d;
   a.QTRC = io.QTRC; a.QTRC0 = io.QTRC0; a.RHOQ_t = io.RHOQ_t; a.DENS0 = io.DENS0; a.DENS = io.DENS;
@@ -473,6 +477,7 @@ hipError_t tracer_stage(const Ctx& c, const TracerIO& io, hipStream_t s) {
   a.RCDZ = c.g1.RCDZ; a.RCDX = c.g1.RCDX; a.RCDY = c.g1.RCDY;
   a.dtl = io.dtl; a.QTRCo = io.QTRCo;
   a.phi_lo = c.scr[0]; a.rjpls = c.scr[1]; a.rjmns = c.scr[2];
+  a.dens_mode = io.dens_mode;
   const bool fct = io.flag_fct != 0, along = io.flag_along != 0;
   if (c.scheme_tracer == UD3) return c.terrain ? tracer_t<UD3, true>(c, a, fct, along, s) : tracer_t<UD3, false>(c, a, fct, along, s);
   if (c.scheme_tracer == UD3KOREN)

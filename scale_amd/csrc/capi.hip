@@ -869,8 +869,7 @@ int scale_hip_model_create(scale_hip_ctx* h, const scale_hip_dyn_config* cfg, in
     for (int v = 0; v < 5; ++v) M->R[r][v] = A(n3);
     M->mfR[r] = A(3 * n3); M->tfR[r] = A(3 * n3);
   }
-  M->ndq = A(3 * n3); M->DENS_RK = A(n3); M->QRK1 = A(n3); M->QRK2 = A(n3);
-  if (QA > 0 && cfg->tinteg_tracer == SCALE_HIP_TRACER_RK3WS2002) M->DENS_RK2 = A(n3);
+  M->ndq = A(3 * n3); M->QRK1 = A(n3); M->QRK2 = A(n3);
   if (cfg->mixed_precision) {
     M->mixed = 1;
     auto F = [&](size_t n) { return (float*)dalloc(c, (n + 1) / 2, &M->allocs); };
@@ -1001,7 +1000,8 @@ int scale_hip_model_large_step(scale_hip_ctx* h, int32_t n) {
     CK(shp::model_state_to_f64(h->c, shp::F64_DENS | shp::F64_RHOT));  // the preparation reads them
     CK(shp::model_large_step(h->c));
   }
-  CK(shp::model_state_to_f64(h->c));
+  // (with tracers the last step left the density)
+  CK(shp::model_state_to_f64(h->c, n > 0 && h->c.model->QA > 0 ? shp::F64_ALL & ~shp::F64_DENS : shp::F64_ALL));
   shp::prof_stop(h->c, h->c.stream);
   return 0;
 }

@@ -396,10 +396,11 @@ __global__ void axpy_interior(Dims d, double* y, const double* x, double scale_d
   else y[p] = x[p] / scale_div;
 }
 
-// av += f on the interior, the three components of a mass flux in one launch
-// (blockIdx.z = j + JMAX * component)
+// the running mean of a mass flux over the short steps on the interior: the
+// sum av starts at the first and the last stores sum / nstep, three components
+// in one launch (blockIdx.z = j + JMAX * component)
 template <typename R>
-__global__ void mflx_sum(Dims d, double* av, const R* f) {
+__global__ void mflx_mean(Dims d, double* mean, double* av, const R* f, int first, int last, double nstep) {
   const int jmax = d.JE - d.JS + 1;
   const int i = d.IS + blockIdx.x * 64 + threadIdx.x;
   const int k = d.KS + blockIdx.y * 4 + threadIdx.y;
@@ -407,18 +408,9 @@ __global__ void mflx_sum(Dims d, double* av, const R* f) {
   const size_t comp = blockIdx.z / jmax;
   if (i > d.IE || k > d.KE) return;
   const size_t p = IX(d, k, i, j) + d.n3 * comp;
-  av[p] = av[p] + (double)f[p];
-}
-// mflx = av / nstep on the interior, three components in one launch
-__global__ void mflx_mean(Dims d, double* mflx, const double* av, double nstep) {
-  const int jmax = d.JE - d.JS + 1;
-  const int i = d.IS + blockIdx.x * 64 + threadIdx.x;
-  const int k = d.KS + blockIdx.y * 4 + threadIdx.y;
-  const int j = d.JS + (int)(blockIdx.z % jmax);
-  const size_t comp = blockIdx.z / jmax;
-  if (i > d.IE || k > d.KE) return;
-  const size_t p = IX(d, k, i, j) + d.n3 * comp;
-  mflx[p] = av[p] / nstep;
+  const double s = (first ? 0.0 : av[p]) + (double)f[p];
+  if (last) mean[p] = s / nstep;
+  else av[p] = s;
 }
 
 // FP64 budget: per-block partial sums of a*CDZ*CDX*CDY*GSQRT/(MAPF1*MAPF2), fixed order
@@ -729,7 +721,6 @@ hipError_t model_prepare(Ctx& c) {
   hipLaunchKernelGGL(large_prep, grid_full(d), dim3(64, 4), 0, s, d, M.RHOT, M.REF_pres, M.RT2P, M.DPRES0, M.REF_rhot);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(M.DENS00, M.DENS, bytes, hipMemcpyDeviceToDevice, s));
-  HIPCHK(fill_zero(M.mflx_av, 3 * d.n3, s));
   return model_prepare_tend(c);
 }
 
@@ -749,18 +740,25 @@ static hipError_t large_begin(Ctx& c, const StepRec* rec) {
   return hipSuccess;
 }
 
-// after each short step: the sum of the mass fluxes over the short steps
-// (LARGE.F90:960-970), the three components in one launch (in mixed
-// precision from the FP32 fluxes, widened on the fly)
-static hipError_t large_after_short(Ctx& c) {
+// after each short step: the mean of the mass fluxes over the short steps
+// (LARGE.F90:960-970, 1016-1030), which only the tracers read, the three
+// components in one launch (in mixed precision from the FP32 fluxes, widened
+// on the fly).  The first step starts the sum and the last leaves the mean in
+// mflx_hi; the FP64 flux of a single short step is its mean (clearing the sum,
+// adding to it and dividing took 0.29 ms at 320x320x96, and 0.55 ms in mixed
+// precision at 512x384x96, where the one pass left takes 0.15).
+static hipError_t large_after_short(Ctx& c, int step, int nstep) {
   Model& M = *c.model;
   const Dims& d = c.d;
-  if (M.mixed) {
-    if (M.QA <= 0) return hipSuccess;  // only the tracers read the sum
-    hipLaunchKernelGGL(mflx_sum<float>, grid_int3(d), dim3(64, 4), 0, c.stream, d, M.mflx_av, (const float*)M.fmflx);
-  } else {
-    hipLaunchKernelGGL(mflx_sum<double>, grid_int3(d), dim3(64, 4), 0, c.stream, d, M.mflx_av, (const double*)M.mflx_hi);
-  }
+  if (M.QA <= 0 || (nstep == 1 && !M.mixed)) return hipSuccess;
+  const int first = step == 0, last = step == nstep - 1;
+  const double ns = (double)nstep;
+  if (M.mixed)
+    hipLaunchKernelGGL(mflx_mean<float>, grid_int3(d), dim3(64, 4), 0, c.stream, d, M.mflx_hi, M.mflx_av,
+                       (const float*)M.fmflx, first, last, ns);
+  else
+    hipLaunchKernelGGL(mflx_mean<double>, grid_int3(d), dim3(64, 4), 0, c.stream, d, M.mflx_hi, M.mflx_av,
+                       (const double*)M.mflx_hi, first, last, ns);
   return hipGetLastError();
 }
 
@@ -774,17 +772,15 @@ static hipError_t copy_levels(const Ctx& c, double* dst, const double* src, hipS
 
 // the tracers of the large step with the mass flux averaged over its nstep
 // short steps (LARGE.F90:1016-1127)
-static hipError_t large_tracers(Ctx& c, int nstep) {
+static hipError_t large_tracers(Ctx& c) {
   Model& M = *c.model;
   const Dims& d = c.d;
   hipStream_t s = c.stream;
   const double dtl = M.dtl;
   if (M.QA <= 0) return hipSuccess;
   // mixed precision: the tracers advance in FP64 on the FP64 copy of the
-  // end-of-step density and the FP64 sum of the mass fluxes
+  // end-of-step density and the FP64 mean of the mass fluxes
   if (M.mixed) HIPCHK(model_state_to_f64(c, F64_DENS));
-  hipLaunchKernelGGL(mflx_mean, grid_int3(d), dim3(64, 4), 0, s, d, M.mflx_hi, (const double*)M.mflx_av, (double)nstep);
-  HIPCHK(hipGetLastError());
   double* mf[3] = {M.mflx_hi, M.mflx_hi + d.n3, M.mflx_hi + 2 * d.n3};
   HIPCHK(halo_fill(c, mf, 3, s));
   for (int iq = 0; iq < M.QA; ++iq) {
@@ -832,9 +828,9 @@ hipError_t model_large_step(Ctx& c, const StepRec* rec) {
   HIPCHK(large_begin(c, rec));
   for (int step = 0; step < nstep; ++step) {
     HIPCHK(model_short_step_rk4(c, dts, rec));
-    HIPCHK(large_after_short(c));
+    HIPCHK(large_after_short(c, step, nstep));
   }
-  return large_tracers(c, nstep);
+  return large_tracers(c);
 }
 
 // ---- ensembles ---------------------------------------------------------------------
@@ -904,38 +900,6 @@ static void tab_free(Ensemble::Tab& t) {
   t = Ensemble::Tab{};
 }
 
-// ---- ensemble tracers: point tables ---------------------------------------------
-// the preparation of the tracer stages of one member: the mean mass flux
-// (LARGE.F90:1016-1027) on the interior and the two RK3 stage densities on
-// the interior and its one-cell ring, as mflx_mean and dens_rk do
-struct TrPrepEnt {
-  Dims d;
-  double* mflx;
-  const double* av;
-  double nstep;
-  double *rk1, *rk2;
-  const double *D00, *D;
-};
-__global__ void __launch_bounds__(256) tr_prep_batch(const TrPrepEnt* __restrict__ tab, const unsigned* __restrict__ first,
-                                                     int nmem) {
-  const unsigned lt = blockIdx.x;
-  const int m = batch_member(first, nmem, lt);
-  const TrPrepEnt& e = tab[m];
-  const Dims& d = e.d;
-  const int ri = d.IE - d.IS + 3, rj = d.JE - d.JS + 3;
-  const size_t t = (size_t)(lt - first[m]) * 256 + threadIdx.x;
-  const size_t np = (size_t)ri * rj * (size_t)(d.KE - d.KS + 1);
-  if (t >= np) return;
-  const int i = d.IS - 1 + (int)(t % (size_t)ri);
-  const int j = d.JS - 1 + (int)((t / (size_t)ri) % (size_t)rj);
-  const int k = d.KS + (int)(t / ((size_t)ri * rj));
-  const size_t p = IX(d, k, i, j);
-  const double d0 = e.D00[p], d1 = e.D[p];
-  e.rk1[p] = d0 + (d1 - d0) / 3.0;
-  e.rk2[p] = d0 + (d1 - d0) * 0.5;
-  if (i >= d.IS && i <= d.IE && j >= d.JS && j <= d.JE)
-    for (int c = 0; c < 3; ++c) e.mflx[p + d.n3 * c] = e.av[p + d.n3 * c] / e.nstep;
-}
 // a stage's output back into the tracer, levels KS..KE (copy_levels)
 struct CopyEnt {
   double* dst;
@@ -974,12 +938,12 @@ static const unsigned* point_first(const Ensemble::Tab& t) {
 // the start of the large step of every member (large_begin without records,
 // the tendencies aside): in mixed precision the FP64 DENS and RHOT from the
 // FP32 state (from_dev32), then RT2P, DPRES0, REF_rhot (large_prep), DENS00 =
-// DENS and the flux sum cleared; one thread per point of the whole array
+// DENS; one thread per point of the whole array
 struct BeginEnt {
   Dims d;
   const float *fD, *fR;  // mixed precision (else null)
   const double* off;     // their level profiles (DENS, then RHOT)
-  double *DENS, *RHOT, *DENS00, *mflx_av;
+  double *DENS, *RHOT, *DENS00;
   const double* REF_pres;
   double *RT2P, *DPRES0, *REF_rhot;
 };
@@ -1007,16 +971,16 @@ __global__ void __launch_bounds__(256) begin_batch(const BeginEnt* __restrict__ 
   };
   large_prep_point(d, k, i, j, rhot, e.REF_pres, e.RT2P, e.DPRES0, e.REF_rhot);
   e.DENS00[q] = D;
-  for (int c = 0; c < 3; ++c) e.mflx_av[q + d.n3 * c] = 0.0;
 }
-// the flux sum after each short step (large_after_short) of every member
+// the flux mean after each short step (large_after_short) of every member
 struct SumEnt {
   Dims d;
-  double* av;
+  double *mean, *av;
   const float* f32;
   const double* f64;
 };
-__global__ void __launch_bounds__(256) sum_batch(const SumEnt* __restrict__ tab, const unsigned* __restrict__ first, int nmem) {
+__global__ void __launch_bounds__(256) sum_batch(const SumEnt* __restrict__ tab, const unsigned* __restrict__ first, int nmem,
+                                                 int begin, int last, double nstep) {
   const unsigned lt = blockIdx.x;
   const int m = batch_member(first, nmem, lt);
   const SumEnt& e = tab[m];
@@ -1030,7 +994,9 @@ __global__ void __launch_bounds__(256) sum_batch(const SumEnt* __restrict__ tab,
   const size_t p = IX(d, k, i, j);
   for (int c = 0; c < 3; ++c) {
     const size_t q = p + d.n3 * c;
-    e.av[q] = e.av[q] + (e.f32 ? (double)e.f32[q] : e.f64[q]);
+    const double s = (begin ? 0.0 : e.av[q]) + (e.f32 ? (double)e.f32[q] : e.f64[q]);
+    if (last) e.mean[q] = s / nstep;
+    else e.av[q] = s;
   }
 }
 static hipError_t ensemble_begin_build(Ensemble& E) {
@@ -1044,12 +1010,12 @@ static hipError_t ensemble_begin_build(Ensemble& E) {
     BeginEnt b{};
     b.d = d;
     if (M.mixed) { b.fD = M.fS[0]; b.fR = M.fS[4]; b.off = M.foff; }
-    b.DENS = M.DENS; b.RHOT = M.RHOT; b.DENS00 = M.DENS00; b.mflx_av = M.mflx_av;
+    b.DENS = M.DENS; b.RHOT = M.RHOT; b.DENS00 = M.DENS00;
     b.REF_pres = M.REF_pres; b.RT2P = M.RT2P; b.DPRES0 = M.DPRES0; b.REF_rhot = M.REF_rhot;
     be.push_back(b);
     bb.push_back((unsigned)((d.n3 + 255) / 256));
-    if (M.mixed && M.QA <= 0) continue;  // only the tracers read the sum
-    SumEnt e{d, M.mflx_av, M.mixed ? (const float*)M.fmflx : nullptr, M.mixed ? nullptr : (const double*)M.mflx_hi};
+    if (M.QA <= 0 || (!M.mixed && model_nstep(M) == 1)) continue;
+    SumEnt e{d, M.mflx_hi, M.mflx_av, M.mixed ? (const float*)M.fmflx : nullptr, M.mixed ? nullptr : (const double*)M.mflx_hi};
     se.push_back(e);
     sb.push_back((unsigned)(((size_t)(d.IE - d.IS + 1) * (d.JE - d.JS + 1) * (d.KE - d.KS + 1) + 255) / 256));
   }
@@ -1075,10 +1041,10 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
   const int n = (int)E.members.size();
   std::vector<const Ctx*> cs;
   for (Ctx* cp : E.members) cs.push_back(cp);
-  // the FCT stage on LDS tiles for the two-cell schemes (the tiles of all
+  // every stage on LDS tiles for the two-cell schemes (the tiles of all
   // members keep every CU busy even where one member's would not)
   const int st = E.members[0]->scheme_tracer;
-  E.tr_tile = M0.fct && (st == UD3 || st == CD4 || st == UD3KOREN || st == UD1 || st == CD2);
+  E.tr_tile = (st == UD3 || st == CD4 || st == UD3KOREN || st == UD1 || st == CD2);
   for (const Ctx* cp : cs) E.tr_tile = E.tr_tile && cp->d.n3 < TILE_MAX_N3;
   for (auto* v : {&E.tr_s1, &E.tr_s2, &E.tr_ph, &E.tr_s3})
     for (auto& b : *v) batch_free(b);
@@ -1099,22 +1065,24 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
       const double* rq = M.RHOQ_tp ? M.RHOQ_tp + d.n3 * (size_t)iq : nullptr;
       TracerIO io{};  // no tracer filter in the batched case: num_diff_q is zero (null)
       io.RHOQ_t = rq; io.DENS0 = M.DENS00; io.mflx_hi = M.mflx_hi; io.num_diff = nullptr; io.flag_along = M.fct_along;
-      io.QTRCo = M.QRK1; io.QTRC = q; io.QTRC0 = q; io.DENS = M.DENS_RK; io.dtl = M.dtl / 3.0; io.flag_fct = 0;
+      io.QTRCo = M.QRK1; io.QTRC = q; io.QTRC0 = q; io.DENS = M.DENS; io.dens_mode = 1; io.dtl = M.dtl / 3.0; io.flag_fct = 0;
       s1.push_back(io);
-      io.QTRCo = M.QRK2; io.QTRC = M.QRK1; io.DENS = M.DENS_RK2; io.dtl = M.dtl / 2.0;
+      io.QTRCo = M.QRK2; io.QTRC = M.QRK1; io.dens_mode = 2; io.dtl = M.dtl / 2.0;
       s2.push_back(io);
-      io.QTRCo = M.QRK1; io.QTRC = M.QRK2; io.DENS = M.DENS; io.dtl = M.dtl; io.flag_fct = M.fct;
+      io.QTRCo = M.QRK1; io.QTRC = M.QRK2; io.dens_mode = 0; io.dtl = M.dtl; io.flag_fct = M.fct;
       s3.push_back(io);
       const size_t off = d.pl * (size_t)d.KS, nn = d.pl * (size_t)(d.KE - d.KS + 1);
       cp_ents.push_back(CopyEnt{q + off, M.QRK1 + off, nn});
       cp_blocks.push_back((unsigned)((nn + 1023) / 1024));
       qf.push_back({cp, q});
     }
-    HIPCHK(tracer_batch_build(cs.data(), s1.data(), n, false, E.tr_s1[(size_t)iq]));
-    HIPCHK(tracer_batch_build(cs.data(), s2.data(), n, false, E.tr_s2[(size_t)iq]));
     if (E.tr_tile) {
+      HIPCHK(trt_batch_build(cs.data(), s1.data(), n, E.tr_s1[(size_t)iq]));
+      HIPCHK(trt_batch_build(cs.data(), s2.data(), n, E.tr_s2[(size_t)iq]));
       HIPCHK(trt_batch_build(cs.data(), s3.data(), n, E.tr_s3[(size_t)iq]));
     } else {
+      HIPCHK(tracer_batch_build(cs.data(), s1.data(), n, false, E.tr_s1[(size_t)iq]));
+      HIPCHK(tracer_batch_build(cs.data(), s2.data(), n, false, E.tr_s2[(size_t)iq]));
       HIPCHK(tracer_batch_build(cs.data(), s3.data(), n, true, E.tr_ph[(size_t)iq]));
       HIPCHK(tracer_batch_build(cs.data(), s3.data(), n, false, E.tr_s3[(size_t)iq]));
     }
@@ -1122,8 +1090,6 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
     HIPCHK(halo_table<double>(E.tr_q[(size_t)iq], qf));
   }
   std::vector<std::pair<const Ctx*, double*>> mf, q1, q2, rr;
-  std::vector<TrPrepEnt> prep;
-  std::vector<unsigned> prep_blocks;
   for (Ctx* cp : E.members) {
     Model& M = *cp->model;
     const Dims& d = cp->d;
@@ -1132,15 +1098,11 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
     q2.push_back({cp, M.QRK2});
     rr.push_back({cp, cp->scr[1]});
     rr.push_back({cp, cp->scr[2]});
-    prep.push_back(TrPrepEnt{d, M.mflx_hi, M.mflx_av, (double)model_nstep(M), M.DENS_RK, M.DENS_RK2, M.DENS00, M.DENS});
-    const size_t np = (size_t)(d.IE - d.IS + 3) * (size_t)(d.JE - d.JS + 3) * (size_t)(d.KE - d.KS + 1);
-    prep_blocks.push_back((unsigned)((np + 255) / 256));
   }
   HIPCHK(halo_table<double>(E.tr_mf, mf));
   HIPCHK(halo_table<double>(E.tr_q1, q1));
   HIPCHK(halo_table<double>(E.tr_q2, q2));
   HIPCHK(halo_table<double>(E.tr_r, rr));
-  HIPCHK(point_table(E.tr_prep, prep, prep_blocks));
   E.tr_qa = qa; E.tr_fct = M0.fct;
   E.tr_batched = true;
   return hipSuccess;
@@ -1149,14 +1111,12 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
 // the tracers of every member (large_tracers, batched): the preparation,
 // then per tracer the three stages, each with the halo fill of its output
 static hipError_t ensemble_tracers(Ensemble& E, hipStream_t s) {
-  hipLaunchKernelGGL(tr_prep_batch, dim3(E.tr_prep.total), dim3(256), 0, s, (const TrPrepEnt*)E.tr_prep.dev,
-                     point_first<TrPrepEnt>(E.tr_prep), E.tr_prep.n);
-  HIPCHK(hipGetLastError());
   HIPCHK(halo_table_launch<double>(E.tr_mf, s));
   for (int iq = 0; iq < E.tr_qa; ++iq) {
-    HIPCHK(tracer_batch_launch(E.tr_s1[(size_t)iq], 0, s));  // stage 1: dt/3, no FCT
+    auto nofct = [&](const BatchBuf& b) { return E.tr_tile ? trt_batch_launch(b, 2, s) : tracer_batch_launch(b, 0, s); };
+    HIPCHK(nofct(E.tr_s1[(size_t)iq]));  // stage 1: dt/3, no FCT
     HIPCHK(halo_table_launch<double>(E.tr_q1, s));
-    HIPCHK(tracer_batch_launch(E.tr_s2[(size_t)iq], 0, s));  // stage 2: dt/2, no FCT
+    HIPCHK(nofct(E.tr_s2[(size_t)iq]));  // stage 2: dt/2, no FCT
     HIPCHK(halo_table_launch<double>(E.tr_q2, s));
     if (E.tr_fct && E.tr_tile) {  // stage 3: dt, FCT on tiles
       HIPCHK(trt_batch_launch(E.tr_s3[(size_t)iq], 0, s));
@@ -1168,7 +1128,7 @@ static hipError_t ensemble_tracers(Ensemble& E, hipStream_t s) {
       HIPCHK(halo_table_launch<double>(E.tr_r, s));
       HIPCHK(tracer_batch_launch(E.tr_s3[(size_t)iq], 3, s));
     } else {
-      HIPCHK(tracer_batch_launch(E.tr_s3[(size_t)iq], 0, s));
+      HIPCHK(nofct(E.tr_s3[(size_t)iq]));
     }
     const Ensemble::Tab& t = E.tr_copy[(size_t)iq];
     hipLaunchKernelGGL(copy_batch, dim3(t.total), dim3(256), 0, s, (const CopyEnt*)t.dev, point_first<CopyEnt>(t), t.n);
@@ -1251,18 +1211,10 @@ static hipError_t ensemble_step_t(Ensemble& E) {
     return hipSuccess;
   };
   // the preparation of every member (reading the FP64 DENS and RHOT, refreshed
-  // from the FP32 state in mixed precision) in one launch; the tendencies on
-  // the lanes where they are (re)computed
+  // from the FP32 state in mixed precision) in one launch
   hipLaunchKernelGGL(begin_batch, dim3(E.begin.total), dim3(256), 0, s, (const BeginEnt*)E.begin.dev,
                      point_first<BeginEnt>(E.begin), E.begin.n);
   HIPCHK(hipGetLastError());
-  bool tend = false;
-  for (Ctx* cp : E.members) tend = tend || tend_needed(*cp->model);
-  if (tend) {
-    HIPCHK(fork());
-    for (Ctx* cp : E.members) HIPCHK(model_prepare_tend(*cp));
-    HIPCHK(join());
-  }
   for (int step = 0; step < nstep; ++step) {
     // numerical filter (LARGE.F90:845-858) and its halos: one launch each
     // (a member with ND_COEF = 0 gets zeros)
@@ -1277,15 +1229,15 @@ static hipError_t ensemble_step_t(Ensemble& E) {
       HIPCHK(hevi_batch_launch(E.stage[r], E.stage_bpc, E.ncu, s));
       HIPCHK(halo_table_launch<R>(E.halo[r + 1], s));
     }
-    if (E.sum.dev) {  // the flux sums of every member
+    if (E.sum.dev) {  // the flux means of every member
       hipLaunchKernelGGL(sum_batch, dim3(E.sum.total), dim3(256), 0, s, (const SumEnt*)E.sum.dev, point_first<SumEnt>(E.sum),
-                         E.sum.n);
+                         E.sum.n, (int)(step == 0), (int)(step == nstep - 1), (double)nstep);
       HIPCHK(hipGetLastError());
     }
   }
   if (!E.tr_batched) {
     HIPCHK(fork());
-    for (Ctx* cp : E.members) HIPCHK(large_tracers(*cp, nstep));
+    for (Ctx* cp : E.members) HIPCHK(large_tracers(*cp));
     return join();
   }
   if (E.members[0]->model->mixed) {  // the tracers advance on the FP64 copy of the density
@@ -1296,13 +1248,32 @@ static hipError_t ensemble_step_t(Ensemble& E) {
   return ensemble_tracers(E, s);
 }
 
-// every member's FP64 copies of its FP32 state and fluxes (mixed precision),
-// as scale_hip_model_large_step leaves them
-static hipError_t ensemble_finish(Ensemble& E) {
+// the members' tendencies where they are (re)computed, on the lanes: apart
+// from the step, so that a captured step holds none of it (30 launches and
+// their conversions a replay for six members without tendencies)
+static hipError_t ensemble_tend(Ensemble& E) {
+  bool tend = false;
+  for (Ctx* cp : E.members) tend = tend || tend_needed(*cp->model);
+  if (!tend) return hipSuccess;
   hipStream_t s = E.stream;
   HIPCHK(hipEventRecord(E.ev_main, s));
   for (int l = 0; l < E.nlanes; ++l) HIPCHK(hipStreamWaitEvent(E.lane[l], E.ev_main, 0));
-  for (Ctx* cp : E.members) HIPCHK(model_state_to_f64(*cp));
+  for (Ctx* cp : E.members) HIPCHK(model_prepare_tend(*cp));
+  for (int l = 0; l < E.nlanes; ++l) {
+    HIPCHK(hipEventRecord(E.ev_lane[l], E.lane[l]));
+    HIPCHK(hipStreamWaitEvent(s, E.ev_lane[l], 0));
+  }
+  return hipSuccess;
+}
+
+// every member's FP64 copies of its FP32 state and fluxes (mixed precision),
+// as scale_hip_model_large_step leaves them
+static hipError_t ensemble_finish(Ensemble& E, bool stepped) {
+  hipStream_t s = E.stream;
+  HIPCHK(hipEventRecord(E.ev_main, s));
+  for (int l = 0; l < E.nlanes; ++l) HIPCHK(hipStreamWaitEvent(E.lane[l], E.ev_main, 0));
+  // (with tracers the last step left the density)
+  for (Ctx* cp : E.members) HIPCHK(model_state_to_f64(*cp, cp->model->QA > 0 && stepped ? F64_ALL & ~F64_DENS : F64_ALL));
   for (int l = 0; l < E.nlanes; ++l) {
     HIPCHK(hipEventRecord(E.ev_lane[l], E.lane[l]));
     HIPCHK(hipStreamWaitEvent(s, E.ev_lane[l], 0));
@@ -1338,6 +1309,7 @@ hipError_t ensemble_large_step(Ensemble& E, int n) {
   for (Ctx* cp : E.members) HIPCHK(hipStreamSynchronize(cp->stream));
   MemberStreams guard(E);
   for (int q = 0; q < n; ++q) {
+    HIPCHK(ensemble_tend(E));
     if (!E.use_graph) {
       HIPCHK(ensemble_step_direct(E));
       continue;
@@ -1354,7 +1326,7 @@ hipError_t ensemble_large_step(Ensemble& E, int n) {
     }
     HIPCHK(hipGraphLaunch(E.exec, E.stream));
   }
-  return E.members[0]->model->mixed ? ensemble_finish(E) : hipSuccess;
+  return E.members[0]->model->mixed ? ensemble_finish(E, n > 0) : hipSuccess;
 }
 
 void ensemble_free(Ensemble& E) {
@@ -1374,7 +1346,7 @@ void ensemble_free(Ensemble& E) {
     for (auto& b : *v) batch_free(b);
     v->clear();
   }
-  for (auto* t : {&E.tr_mf, &E.tr_q1, &E.tr_q2, &E.tr_r, &E.tr_prep, &E.begin, &E.sum}) tab_free(*t);
+  for (auto* t : {&E.tr_mf, &E.tr_q1, &E.tr_q2, &E.tr_r, &E.begin, &E.sum}) tab_free(*t);
   for (auto* v : {&E.tr_q, &E.tr_copy}) {
     for (auto& t : *v) tab_free(t);
     v->clear();

@@ -25,8 +25,7 @@ struct Model {
   double* S0[5] = {};
   double* R[4][5] = {};
   double *mfR[4] = {}, *tfR[4] = {};
-  double *ndq = nullptr, *DENS_RK = nullptr, *QRK1 = nullptr, *QRK2 = nullptr;
-  double* DENS_RK2 = nullptr;  // the second RK3 tracer stage's density (DENS_RK holds the first's)
+  double *ndq = nullptr, *QRK1 = nullptr, *QRK2 = nullptr;
   // mixed precision: FP32 state, stage, tendency, filter and flux arrays
   // (the FP64 arrays above keep the reference state, the pressure terms and
   // a copy of the state for the large-step preparation and the budgets)
@@ -84,12 +83,12 @@ struct Ensemble {
   // the same number of tracers, the RK3 tracer integration, no tracer filter,
   // one FCT setting and one two-cell tracer scheme: per tracer the tables of
   // stages 1 and 2, of the FCT phi_lo pass and of the last stage; halo tables
-  // of the mass fluxes, QRK1, QRK2, R+/R- and each tracer; the point tables
-  // of the preparation (flux mean, stage densities) and of each copy back
+  // of the mass fluxes, QRK1, QRK2, R+/R- and each tracer; the point table of
+  // each copy back
   bool tr_batched = false, tr_tile = false;
   int tr_qa = 0, tr_fct = 0;
   std::vector<BatchBuf> tr_s1, tr_s2, tr_ph, tr_s3;
-  Tab tr_mf, tr_q1, tr_q2, tr_r, tr_prep;
+  Tab tr_mf, tr_q1, tr_q2, tr_r;
   std::vector<Tab> tr_q, tr_copy;
   bool built = false;
   // lanes: streams the members' own launches spread over (member m on lane

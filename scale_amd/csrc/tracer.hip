@@ -367,6 +367,7 @@ hipError_t tracer_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, 
     a.RCDZ = c.g1.RCDZ; a.RCDX = c.g1.RCDX; a.RCDY = c.g1.RCDY;
     a.dtl = io.dtl; a.QTRCo = io.QTRCo;
     a.phi_lo = c.scr[0]; a.rjpls = c.scr[1]; a.rjmns = c.scr[2];
+    a.dens_mode = io.dens_mode;
     const Dims& d = c.d;
     const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1, kmax = d.KE - d.KS + 1;
     const unsigned ni_t = philo ? (imax + 2 + 63) / 64 : (imax + 63) / 64, nk_t = (kmax + 3) / 4;

@@ -461,8 +461,8 @@ __global__ void __launch_bounds__(64 * TJ) trt_update(TtArgs a, unsigned ni_tile
   trt_update_body<S, TJ, LIM, TER>(a, lb % ntile, ni_tiles, k0, min(a.d.KE, k0 + L - 1));
 }
 
-// both passes over the tiles of many members (batch.h tables; ni[m] the
-// member's tiles across)
+// the passes over the tiles of many members (batch.h tables; ni[m] the
+// member's tiles across): kinds 0 R+/R-, 1 the update, 2 the stage without FCT
 template <int KIND, int S, int TJ, bool VECT>
 __global__ void __launch_bounds__(64 * TJ) trt_batch(const TtArgs* __restrict__ tab, const unsigned* __restrict__ first,
                                                      const unsigned* __restrict__ ni, int nmem, unsigned total) {
@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(64 * TJ) trt_batch(const TtArgs* __restrict__ 
     const int m = batch_member(first, nmem, lt);
     const Dims& d = tab[m].d;
     if constexpr (KIND == 0) trt_ratio_body<S, TJ, VECT, false>(tab[m], lt - first[m], ni[m], d.KS, d.KE);
-    else trt_update_body<S, TJ, true, false>(tab[m], lt - first[m], ni[m], d.KS, d.KE);
+    else trt_update_body<S, TJ, KIND == 1, false>(tab[m], lt - first[m], ni[m], d.KS, d.KE);
     __syncthreads();
   }
 }
@@ -559,7 +559,7 @@ hipError_t tracer_stage_tile(const Ctx& c, const TracerIO& io, double* rjpls, do
   }
 }
 
-// the FCT passes of every member on tiles (the members' stage-3 arguments;
+// the stages of every member on tiles (the members' stage arguments;
 // flat terrain, one two-cell scheme, one bound kind)
 hipError_t trt_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, BatchBuf& b) {
   if (n <= 0) return hipErrorInvalidValue;
@@ -579,7 +579,7 @@ hipError_t trt_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, Bat
     a.RCDZ = c.g1.RCDZ; a.RCDX = c.g1.RCDX; a.RCDY = c.g1.RCDY;
     a.dtl = io.dtl; a.QTRCo = io.QTRCo;
     a.rjpls = c.scr[1]; a.rjmns = c.scr[2];
-    a.GSQRT = nullptr; a.MAPF = nullptr; a.dens_mode = 0;
+    a.GSQRT = nullptr; a.MAPF = nullptr; a.dens_mode = io.dens_mode;
     const Dims& d = c.d;
     ni[(size_t)m] = (unsigned)((d.IE - d.IS + 1 + 63) / 64);
     first[(size_t)m + 1] = first[(size_t)m] + ni[(size_t)m] * (unsigned)((d.JE - d.JS + 1 + TT_TJ - 1) / TT_TJ);
@@ -599,7 +599,7 @@ static hipError_t trt_batch_t(const BatchBuf& b, hipStream_t s) {
   else if (KIND == 0)
     hipLaunchKernelGGL((trt_batch<0, S, TT_TJ, false>), dim3(b.total), dim3(64, TT_TJ), 0, s, tab, first, ni, b.nmem, b.total);
   else
-    hipLaunchKernelGGL((trt_batch<1, S, TT_TJ, false>), dim3(b.total), dim3(64, TT_TJ), 0, s, tab, first, ni, b.nmem, b.total);
+    hipLaunchKernelGGL((trt_batch<KIND == 0 ? 1 : KIND, S, TT_TJ, false>), dim3(b.total), dim3(64, TT_TJ), 0, s, tab, first, ni, b.nmem, b.total);
   return hipGetLastError();
 }
 template <int KIND>
@@ -614,7 +614,7 @@ static hipError_t trt_batch_k(const BatchBuf& b, hipStream_t s) {
 }
 hipError_t trt_batch_launch(const BatchBuf& b, int kind, hipStream_t s) {
   if (!b.dev) return hipErrorInvalidValue;
-  return kind == 0 ? trt_batch_k<0>(b, s) : trt_batch_k<1>(b, s);
+  return kind == 0 ? trt_batch_k<0>(b, s) : kind == 1 ? trt_batch_k<1>(b, s) : trt_batch_k<2>(b, s);
 }
 
 }  // namespace shp

@@ -37,3 +37,39 @@ def test_tendencies_given_later(hip, split, monkeypatch):  # noqa: F811
         for k in hip.STATE:
             ref = later.state[k]
             assert np.abs(ctx.model_get(k) - ref).max() <= 1e-12 * np.abs(ref).max(), k
+
+
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("nstep", [1, 3])
+def test_tendencies_given_to_a_replayed_ensemble(hip, mixed, nstep):  # noqa: F811
+    """An ensemble replaying its captured step is given tendencies: each member
+    stays bit-identical to its own model, with one short step and with three
+    a large step (the mean of the mass fluxes that the tracers take)."""
+    cases = [H.small_case(kmax=10, imax=9, jmax=6, seed=44), H.small_case(kmax=12, imax=66, jmax=5, seed=45)]
+    kw = dict(mixed_precision=mixed, dtl=nstep * 0.5)
+    rng = np.random.Generator(np.random.PCG64(9))
+    tps = []
+    for case in cases:
+        g = case.grid
+        a = g.zeros()
+        a[:, g.IS:g.IE + 1, g.JS:g.JE + 1] = 1e-3 * rng.standard_normal((g.KA, g.imax, g.jmax))
+        tps.append(inputs.halo_fill(g, a))
+    alone = [hip.model_from_case(c, **kw) for c in cases]
+    members = [hip.model_from_case(c, **kw) for c in cases]
+    try:
+        with hip.Ensemble(members) as ens:
+            ens.set_graph(True)
+            for given in (False, True):
+                for ctx, tp in zip(alone + members, tps + tps):
+                    if given:
+                        ctx.model_set("RHOT_tp", tp)
+                for ctx in alone:
+                    ctx.model_large_step(2)
+                ens.large_step(2)
+                ens.synchronize()
+                for case, x, y in zip(cases, alone, members):
+                    for f in hip.STATE + ("mflx_hi",) + tuple(hip.QTRC_BASE + n for n in range(case.qtrc.shape[-1])):
+                        assert np.array_equal(x.model_get(f), y.model_get(f)), (given, f)
+    finally:
+        for ctx in alone + members:
+            ctx.close()

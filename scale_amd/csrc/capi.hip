@@ -4,16 +4,42 @@
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
+#include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 #include "../../include/scale_hip.h"
 #include "common.h"
 #include "model.h"
 #include "shp_internal.h"
 
+// pinned slots through which a call's arrays cross the bus (allocated on first use)
+struct HostPipe {
+  static constexpr int SLOTS = 8;
+  static constexpr size_t SLOT = (size_t)4 << 20;
+  char* buf = nullptr;
+  hipEvent_t ev[SLOTS] = {};
+  char* slot(size_t q) { return buf + (q % SLOTS) * SLOT; }
+  hipError_t init() {
+    if (buf) return hipSuccess;
+    for (auto& e : ev)
+      if (!e)
+        if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return r;
+    return hipHostMalloc((void**)&buf, SLOTS * SLOT, hipHostMallocDefault);
+  }
+  void free() {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (buf) (void)hipHostFree(buf);
+  }
+};
+
 struct scale_hip_ctx {
   shp::Ctx c;
+  HostPipe pipe;
   // drop-in device buffers (allocated on first use)
   std::vector<double*> dbuf;
   bool dropin_ready = false;
@@ -108,10 +134,185 @@ int upload_raw(Ctx& c, double* dst, const double* host, size_t n) {
 }
 
 bool all_equal(const double* a, size_t n, double v) {
-  for (size_t q = 0; q < n; ++q)
-    if (a[q] != v) return false;
+  for (size_t q = 0; q < n;) {  // blocks without an exit, so that the compares vectorise
+    const size_t e = std::min(n, q + 1024);
+    bool ne = false;
+    for (; q < e; ++q) ne |= a[q] != v;
+    if (ne) return false;
+  }
   return true;
 }
+
+// Whether host arrays hold constants (metrics of flat terrain), looked over on
+// threads of the call while it uploads its other arguments; finished before
+// the call returns.  The 200 MB of a 128x128x64 stage's metrics took the
+// calling thread 7 of the call's 28.5 ms; beside the transfers they add
+// nothing.  Less than 2 MB it looks over by itself.
+class ConstCheck {
+ public:
+  ~ConstCheck() { join(); }
+  void add(const double* a, size_t n, double v) {
+    if (!a) bad_ = true;
+    else for (size_t o = 0; o < n; o += BLOCK) parts_.push_back({a + o, std::min(BLOCK, n - o), v});
+  }
+  void start() {
+    if (bad_ || parts_.size() < 16) return;
+    try {
+      for (int t = 0; t < 4; ++t) threads_.emplace_back([this] { work(); });
+    } catch (const std::system_error&) {  // no more threads: result() does the work
+    }
+  }
+  bool result() {
+    work();
+    join();
+    return !bad_;
+  }
+
+ private:
+  struct Part { const double* a; size_t n; double v; };
+  static constexpr size_t BLOCK = 16384;  // 128 KB
+  void work() {
+    for (size_t q; !bad_ && (q = next_++) < parts_.size();)
+      if (!all_equal(parts_[q].a, parts_[q].n, parts_[q].v)) bad_ = true;
+  }
+  void join() {
+    for (auto& t : threads_) t.join();
+    threads_.clear();
+  }
+  std::vector<Part> parts_;
+  std::vector<std::thread> threads_;
+  std::atomic<size_t> next_{0};
+  std::atomic<bool> bad_{false};
+};
+
+// The arrays of one call between host Fortran order and the device layout,
+// in chunks through the pinned slots: threads of the call copy between the
+// caller's memory and the slots while the calling thread, which helps them
+// where it would wait, feeds the DMA engine and the layout kernels.  One
+// thread's copies (what a pageable hipMemcpyAsync does) feed the bus at half
+// its rate: a 128x128x64 stage's 550 MB took 21.7 ms and takes 13.7 (slots of
+// 1 MB, each with its launch and wait, 19.1; seven threads 13.5).  A call of
+// fewer bytes than the threads are worth copies array by array: 21 MB in 1.70
+// ms against 1.80 through the slots, 90 MB in 4.8 against 3.6.
+class ArrayCopy {
+ public:
+  ArrayCopy(Ctx& c, HostPipe& pipe, bool up) : c_(c), pipe_(pipe), up_(up) {}
+  ~ArrayCopy() { join(); }
+  void up(double* dev, const double* host, int ncomp) { add(dev, const_cast<double*>(host), ncomp); }
+  void down(double* host, double* dev, int ncomp) { add(dev, host, ncomp); }
+  int run() {
+    if (null_) return fail("null array argument");
+    if (chunks_.empty()) return 0;
+    // small arrays, or no pinned memory: one after the other
+    if (bytes_ < (up_ ? MIN_UP : MIN_DOWN) || pipe_.init() != hipSuccess) {
+      (void)hipGetLastError();
+      for (const Chunk& k : chunks_) {
+        if (!k.first) continue;
+        const Job& j = jobs_[k.job];
+        if (int r = up_ ? upload3(c_, j.dev, (const double*)k.host, j.ncomp) : download3(c_, (double*)k.host, j.dev, j.ncomp)) return r;
+      }
+      return 0;
+    }
+    if (int r = ensure_stage(c_, stage_)) return r;
+    std::vector<std::atomic<unsigned char>> done(chunks_.size());
+    for (auto& d : done) d.store(0, std::memory_order_relaxed);
+    done_ = done.data();
+    try {
+      for (int t = 0; t < 4; ++t)
+        threads_.emplace_back([this] { while (!stop_ && next_ < chunks_.size()) if (!copy_one()) std::this_thread::yield(); });
+    } catch (const std::system_error&) {  // no more threads: the caller's copies
+    }
+    const hipError_t e = up_ ? run_up() : run_down();
+    join();
+    if (e != hipSuccess) (void)hipStreamSynchronize(c_.stream);  // the slots are in use until then
+    CK(e);
+    return 0;
+  }
+
+ private:
+  static constexpr size_t MIN_UP = (size_t)32 << 20, MIN_DOWN = (size_t)16 << 20;
+  struct Job { double* dev; int ncomp; };
+  struct Chunk { char* host; size_t off, n; size_t job; bool first, last; };  // off, n: bytes of the job's staged array
+  void add(double* dev, double* host, int ncomp) {
+    if (!host) { null_ = true; return; }
+    const size_t total = c_.d.n3 * (size_t)ncomp * sizeof(double);
+    stage_ = std::max(stage_, total / sizeof(double));
+    bytes_ += total;
+    for (size_t o = 0; o < total; o += HostPipe::SLOT) {
+      const size_t n = std::min(HostPipe::SLOT, total - o);
+      chunks_.push_back({(char*)host + o, o, n, jobs_.size(), o == 0, o + n == total});
+    }
+    jobs_.push_back({dev, ncomp});
+  }
+  // copies the next chunk below limit_; false where there is none
+  bool copy_one() {
+    size_t q = next_;
+    do {
+      if (q >= limit_) return false;
+    } while (!next_.compare_exchange_weak(q, q + 1));
+    const Chunk& k = chunks_[q];
+    if (up_) memcpy(pipe_.slot(q), k.host, k.n);
+    else memcpy(k.host, pipe_.slot(q), k.n);
+    done_[q].store(1, std::memory_order_release);
+    return true;
+  }
+  void wait(size_t q) {
+    while (!done_[q].load(std::memory_order_acquire))
+      if (!copy_one()) std::this_thread::yield();
+  }
+  hipError_t run_up() {
+    constexpr size_t SLOTS = HostPipe::SLOTS, AHEAD = SLOTS / 2;  // chunks given to the DMA engine before the first is waited for
+    limit_ = std::min(chunks_.size(), SLOTS);
+    for (size_t q = 0; q < chunks_.size(); ++q) {
+      wait(q);
+      const Chunk& k = chunks_[q];
+      if (hipError_t e = hipMemcpyAsync((char*)c_.stage + k.off, pipe_.slot(q), k.n, hipMemcpyHostToDevice, c_.stream)) return e;
+      if (hipError_t e = hipEventRecord(pipe_.ev[q % SLOTS], c_.stream)) return e;
+      if (k.last)
+        if (hipError_t e = shp::to_device_layout(c_, jobs_[k.job].dev, c_.stage, jobs_[k.job].ncomp, c_.stream)) return e;
+      if (q >= AHEAD) {
+        if (hipError_t e = hipEventSynchronize(pipe_.ev[(q - AHEAD) % SLOTS])) return e;
+        limit_ = std::min(chunks_.size(), q - AHEAD + 1 + SLOTS);
+      }
+    }
+    // the slots are free once the engine has read them
+    return hipEventSynchronize(pipe_.ev[(chunks_.size() - 1) % SLOTS]);
+  }
+  hipError_t run_down() {
+    constexpr size_t SLOTS = HostPipe::SLOTS;
+    size_t issued = 0;
+    for (size_t q = 0; q < chunks_.size(); ++q) {
+      for (; issued < std::min(chunks_.size(), q + SLOTS / 2); ++issued) {
+        if (issued >= SLOTS) wait(issued - SLOTS);
+        const Chunk& k = chunks_[issued];
+        if (k.first)
+          if (hipError_t e = shp::to_fortran_layout(c_, c_.stage, jobs_[k.job].dev, jobs_[k.job].ncomp, c_.stream)) return e;
+        if (hipError_t e = hipMemcpyAsync(pipe_.slot(issued), (char*)c_.stage + k.off, k.n, hipMemcpyDeviceToHost, c_.stream)) return e;
+        if (hipError_t e = hipEventRecord(pipe_.ev[issued % SLOTS], c_.stream)) return e;
+      }
+      if (hipError_t e = hipEventSynchronize(pipe_.ev[q % SLOTS])) return e;
+      limit_ = q + 1;
+    }
+    for (size_t q = 0; q < chunks_.size(); ++q) wait(q);
+    return hipSuccess;
+  }
+  void join() {
+    stop_ = true;
+    for (auto& t : threads_) t.join();
+    threads_.clear();
+  }
+  Ctx& c_;
+  HostPipe& pipe_;
+  const bool up_;
+  bool null_ = false;
+  size_t stage_ = 0, bytes_ = 0;
+  std::vector<Job> jobs_;
+  std::vector<Chunk> chunks_;
+  std::atomic<unsigned char>* done_ = nullptr;
+  std::vector<std::thread> threads_;
+  std::atomic<size_t> next_{0}, limit_{0};
+  std::atomic<bool> stop_{false};
+};
 
 // 1-D grid arrays: CDZ FDZ RCDZ RFDZ (KA) | CDX FDX RCDX RFDX (IA) | CDY FDY RCDY RFDY (JA)
 int set_grid1d(Ctx& c, const double* CDZ, const double* FDZ, const double* RCDZ, const double* RFDZ,
@@ -138,12 +339,21 @@ int set_grid1d(Ctx& c, const double* CDZ, const double* FDZ, const double* RCDZ,
   return 0;
 }
 
+// the metrics of flat terrain
+void flat_check(ConstCheck& k, const Dims& d, const double* GSQRT, const double* J13G, const double* J23G, const double* MAPF) {
+  k.add(MAPF, 8 * d.pl, 1.0);
+  k.add(GSQRT, 7 * d.n3, 1.0);
+  k.add(J13G, 7 * d.n3, 0.0);
+  k.add(J23G, 7 * d.n3, 0.0);
+  k.start();
+}
+
 // metric arrays; decides the flat (TERRAIN=false) specialisation
-int set_metric3d(Ctx& c, const double* PHI, const double* GSQRT, const double* J13G, const double* J23G, double J33G, const double* MAPF) {
+int set_metric3d(Ctx& c, const double* PHI, const double* GSQRT, const double* J13G, const double* J23G, double J33G,
+                 const double* MAPF, ConstCheck& check, HostPipe& pipe) {
   const Dims& d = c.d;
   if (PHI) { if (int r = upload3(c, c.PHI, PHI, 1)) return r; }
-  const bool flat = GSQRT && J13G && J23G && MAPF && all_equal(GSQRT, 7 * d.n3, 1.0) && all_equal(J13G, 7 * d.n3, 0.0) &&
-                    all_equal(J23G, 7 * d.n3, 0.0) && all_equal(MAPF, 8 * d.pl, 1.0);
+  const bool flat = check.result();
   if (!flat) {
     if (!GSQRT || !J13G || !J23G || !MAPF) return fail("metric arrays are required");
     if (!c.GSQRT) {
@@ -152,9 +362,11 @@ int set_metric3d(Ctx& c, const double* PHI, const double* GSQRT, const double* J
       c.J23G = dalloc(c, 7 * d.n3, nullptr);
       if (!c.GSQRT || !c.J13G || !c.J23G) return fail("hipMalloc of metric arrays failed");
     }
-    if (int r = upload3(c, c.GSQRT, GSQRT, 7)) return r;
-    if (int r = upload3(c, c.J13G, J13G, 7)) return r;
-    if (int r = upload3(c, c.J23G, J23G, 7)) return r;
+    ArrayCopy in(c, pipe, true);
+    in.up(c.GSQRT, GSQRT, 7);
+    in.up(c.J13G, J13G, 7);
+    in.up(c.J23G, J23G, 7);
+    if (int r = in.run()) return r;
   }
   if (MAPF) { if (int r = upload_raw(c, c.MAPF, MAPF, 8 * d.pl)) return r; }
   c.terrain = !flat;
@@ -162,6 +374,21 @@ int set_metric3d(Ctx& c, const double* PHI, const double* GSQRT, const double* J
   c.metrics_set = true;
   CK(hipStreamSynchronize(c.stream));
   return 0;
+}
+
+// the metrics of a tracer call (GSQRT and the (IA, JA, 2) map factor); flat
+// terrain leaves the context's metrics as they are
+int set_tracer_metric(Ctx& c, const double* GSQRT, const double* MAPF, ConstCheck& flat, HostPipe& pipe) {
+  const Dims& d = c.d;
+  if (flat.result()) {
+    c.terrain = false;
+    return 0;
+  }
+  if (!GSQRT || !MAPF) return fail("metric arrays are required");
+  std::vector<double> m4(8 * d.pl, 1.0);
+  memcpy(m4.data(), MAPF, 2 * d.pl * sizeof(double));
+  std::vector<double> zero(7 * d.n3, 0.0);
+  return set_metric3d(c, nullptr, GSQRT, zero.data(), zero.data(), 1.0, m4.data(), flat, pipe);
 }
 
 // numerical-filter tables (ATMOS_DYN_filter_setup, COMMON.F90:92-319) and
@@ -386,6 +613,7 @@ int scale_hip_finalize(scale_hip_ctx* h) {
     for (void* q : c.model->allocs) F(q);
     delete c.model;
   }
+  h->pipe.free();
   shp::prof_destroy(c.prof);
   if (c.stream) hipStreamDestroy(c.stream);
   delete h;
@@ -432,28 +660,32 @@ static int short_stage(bool heve, scale_hip_ctx* h,
   if (fct_mom && !c.mfct && !(c.mfct = dalloc(c, shp::MFCT_FIELDS * c.d.n3, nullptr)))
     return fail("hipMalloc failed for the momentum FCT work arrays");
   if (int r = set_grid1d(c, CDZ, FDZ, RCDZ, RFDZ, nullptr, FDX, RCDX, RFDX, nullptr, FDY, RCDY, RFDY)) return r;
-  if (int r = set_metric3d(c, PHI, GSQRT, J13G, J23G, *J33G, MAPF)) return r;
+  ConstCheck flat;
+  flat_check(flat, c.d, GSQRT, J13G, J23G, MAPF);
   auto& B = h->dbuf;
   const double* s0[5] = {DENS0, MOMZ0, MOMX0, MOMY0, RHOT0};
   const double* s[5] = {DENS, MOMZ, MOMX, MOMY, RHOT};
   const double* t[5] = {DENS_t, MOMZ_t, MOMX_t, MOMY_t, RHOT_t};
   double* o[5] = {DENS_RK, MOMZ_RK, MOMX_RK, MOMY_RK, RHOT_RK};
+  ArrayCopy in(c, h->pipe, true);
   for (int v = 0; v < 5; ++v) {
-    if (int r = upload3(c, B[B_S0 + v], s0[v], 1)) return r;
-    if (int r = upload3(c, B[B_S + v], s[v], 1)) return r;
-    if (int r = upload3(c, B[B_T + v], t[v], 1)) return r;
-    if (int r = upload3(c, B[B_OUT + v], o[v], 1)) return r;  // elements HEVI leaves alone keep their values
+    in.up(B[B_S0 + v], s0[v], 1);
+    in.up(B[B_S + v], s[v], 1);
+    in.up(B[B_T + v], t[v], 1);
+    in.up(B[B_OUT + v], o[v], 1);  // elements HEVI leaves alone keep their values
   }
-  if (int r = upload3(c, B[B_DPRES0], DPRES0, 1)) return r;
-  if (int r = upload3(c, B[B_RT2P], RT2P, 1)) return r;
-  if (int r = upload3(c, B[B_REFD], REF_dens, 1)) return r;
-  if (int r = upload3(c, B[B_REFR], REF_rhot, 1)) return r;
-  if (int r = upload3(c, B[B_DDIV], DDIV, 1)) return r;
-  if (int r = upload3(c, B[B_ND], num_diff, 15)) return r;
-  if (int r = upload3(c, B[B_MF], mflx_hi, 3)) return r;
-  if (int r = upload3(c, B[B_TF], tflx_hi, 3)) return r;
+  in.up(B[B_DPRES0], DPRES0, 1);
+  in.up(B[B_RT2P], RT2P, 1);
+  in.up(B[B_REFD], REF_dens, 1);
+  in.up(B[B_REFR], REF_rhot, 1);
+  in.up(B[B_DDIV], DDIV, 1);
+  in.up(B[B_ND], num_diff, 15);
+  in.up(B[B_MF], mflx_hi, 3);
+  in.up(B[B_TF], tflx_hi, 3);
+  if (int r = in.run()) return r;
   if (int r = upload_raw(c, B[B_COR], CORIOLI, c.d.pl)) return r;
   if (int r = upload_raw(c, B[B_WD], wdamp_coef, (size_t)c.d.KA)) return r;
+  if (int r = set_metric3d(c, PHI, GSQRT, J13G, J23G, *J33G, MAPF, flat, h->pipe)) return r;
   const bool has_cor = !all_equal(CORIOLI, c.d.pl, 0.0);
   shp::StageIO io;
   io.ctx = &c;
@@ -466,11 +698,11 @@ static int short_stage(bool heve, scale_hip_ctx* h,
   io.fct_t = heve && FLAG_FCT_T && *FLAG_FCT_T;
   io.fct_along = !FLAG_FCT_ALONG_STREAM || *FLAG_FCT_ALONG_STREAM;
   CK(heve ? shp::heve_stage(io, c.stream) : shp::hevi_stage(io, c.stream));
-  for (int v = 0; v < 5; ++v)
-    if (int r = download3(c, o[v], B[B_OUT + v], 1)) return r;
-  if (int r = download3(c, mflx_hi, B[B_MF], 3)) return r;
-  if (int r = download3(c, tflx_hi, B[B_TF], 3)) return r;
-  return 0;
+  ArrayCopy out(c, h->pipe, false);
+  for (int v = 0; v < 5; ++v) out.down(o[v], B[B_OUT + v], 1);
+  out.down(mflx_hi, B[B_MF], 3);
+  out.down(tflx_hi, B[B_TF], 3);
+  return out.run();
 }
 
 int scale_hip_tstep_short_hevi(scale_hip_ctx* h,
@@ -540,7 +772,9 @@ int scale_hip_tstep_short_hevi_adj(scale_hip_ctx* h,
   if (c.d.IS != 2) return fail("the adjoint supports IHALO = 2 only");
   if (int r = ensure_dropin(h)) return r;
   if (int r = set_grid1d(c, CDZ, FDZ, RCDZ, RFDZ, nullptr, FDX, RCDX, RFDX, nullptr, FDY, RCDY, RFDY)) return r;
-  if (int r = set_metric3d(c, PHI, GSQRT, J13G, J23G, *J33G, MAPF)) return r;
+  ConstCheck flat;
+  flat_check(flat, c.d, GSQRT, J13G, J23G, MAPF);
+  if (int r = set_metric3d(c, PHI, GSQRT, J13G, J23G, *J33G, MAPF, flat, h->pipe)) return r;
   CK(shp::adj_setup(c, 0, 0));
   auto& B = h->dbuf;
   const double* s0[5] = {DENS0, MOMZ0, MOMX0, MOMY0, RHOT0};
@@ -605,15 +839,10 @@ int scale_hip_tstep_tracer_heve(scale_hip_ctx* h,
   if (int r = ensure_dropin(h)) return r;
   if (int r = set_grid1d(c, CDZ, nullptr, RCDZ, nullptr, nullptr, nullptr, RCDX, nullptr, nullptr, nullptr, RCDY, nullptr)) return r;
   // metrics: GSQRT(KA,IA,JA,7) and the (IA,JA,2) map factor
-  const bool flat = all_equal(GSQRT, 7 * d.n3, 1.0) && all_equal(MAPF, 2 * d.pl, 1.0);
-  if (!flat) {
-    std::vector<double> m4(8 * d.pl, 1.0);
-    memcpy(m4.data(), MAPF, 2 * d.pl * sizeof(double));
-    std::vector<double> zero(7 * d.n3, 0.0);
-    if (int r = set_metric3d(c, nullptr, GSQRT, zero.data(), zero.data(), 1.0, m4.data())) return r;
-  } else {
-    c.terrain = false;
-  }
+  ConstCheck flat;
+  flat.add(MAPF, 2 * d.pl, 1.0);
+  flat.add(GSQRT, 7 * d.n3, 1.0);
+  flat.start();
   auto& B = h->dbuf;
   // reuse drop-in buffers: QTRCo, QTRC, QTRC0, RHOQ_t, DENS0, DENS, mflx(3), num_diff(3)
   double* dQo = B[B_OUT]; double* dQ = B[B_S]; double* dQ0 = B[B_S + 1]; double* dRQ = B[B_S + 2];
@@ -626,6 +855,7 @@ int scale_hip_tstep_tracer_heve(scale_hip_ctx* h,
   if (int r = upload3(c, dD, DENS, 1)) return r;
   if (int r = upload3(c, dMF, mflx_hi, 3)) return r;
   if (int r = upload3(c, dND, num_diff, 3)) return r;
+  if (int r = set_tracer_metric(c, GSQRT, MAPF, flat, h->pipe)) return r;
   shp::TracerIO io;
   io.QTRCo = dQo; io.QTRC = dQ; io.QTRC0 = dQ0; io.RHOQ_t = dRQ; io.DENS0 = dD0; io.DENS = dD;
   io.mflx_hi = dMF; io.num_diff = dND; io.dtl = *dtl; io.flag_fct = *FLAG_FCT_TRACER; io.flag_along = *FLAG_FCT_ALONG_STREAM;
@@ -651,15 +881,10 @@ int scale_hip_tstep_tracer_heve_adj(scale_hip_ctx* h,
     return fail("the tracer adjoint needs a face form linear in the tracer; UD3KOREN1993's limiter is not");
   if (int r = ensure_dropin(h)) return r;
   if (int r = set_grid1d(c, CDZ, nullptr, RCDZ, nullptr, nullptr, nullptr, RCDX, nullptr, nullptr, nullptr, RCDY, nullptr)) return r;
-  const bool flat = all_equal(GSQRT, 7 * d.n3, 1.0) && all_equal(MAPF, 2 * d.pl, 1.0);
-  if (!flat) {
-    std::vector<double> m4(8 * d.pl, 1.0);
-    memcpy(m4.data(), MAPF, 2 * d.pl * sizeof(double));
-    std::vector<double> zero(7 * d.n3, 0.0);
-    if (int r = set_metric3d(c, nullptr, GSQRT, zero.data(), zero.data(), 1.0, m4.data())) return r;
-  } else {
-    c.terrain = false;
-  }
+  ConstCheck flat;
+  flat.add(MAPF, 2 * d.pl, 1.0);
+  flat.add(GSQRT, 7 * d.n3, 1.0);
+  flat.start();
   auto& B = h->dbuf;
   // inputs: QTRCo_b, QTRC, QTRC0, DENS0, DENS, mflx(3), num_diff(3); outputs in
   // the tendency buffers and num_diff's components 3..5
@@ -673,6 +898,7 @@ int scale_hip_tstep_tracer_heve_adj(scale_hip_ctx* h,
   if (int r = upload3(c, dD, DENS, 1)) return r;
   if (int r = upload3(c, dMF, mflx_hi, 3)) return r;
   if (int r = upload3(c, dND, num_diff, 3)) return r;
+  if (int r = set_tracer_metric(c, GSQRT, MAPF, flat, h->pipe)) return r;
   shp::TracerIO io{};
   io.QTRC = dQ; io.QTRC0 = dQ0; io.DENS0 = dD0; io.DENS = dD; io.mflx_hi = dMF; io.num_diff = dND;
   io.dtl = *dtl; io.flag_fct = *FLAG_FCT_TRACER; io.flag_along = *FLAG_FCT_ALONG_STREAM;
@@ -778,7 +1004,9 @@ int scale_hip_set_metrics(scale_hip_ctx* h,
   if (!CDZ || !FDZ || !RCDZ || !RFDZ || !CDX || !FDX || !RCDX || !RFDX || !CDY || !FDY || !RCDY || !RFDY)
     return fail("every 1-D grid array is required");
   if (int r = set_grid1d(h->c, CDZ, FDZ, RCDZ, RFDZ, CDX, FDX, RCDX, RFDX, CDY, FDY, RCDY, RFDY)) return r;
-  return set_metric3d(h->c, PHI, GSQRT, J13G, J23G, *J33G, MAPF);
+  ConstCheck flat;
+  flat_check(flat, h->c.d, GSQRT, J13G, J23G, MAPF);
+  return set_metric3d(h->c, PHI, GSQRT, J13G, J23G, *J33G, MAPF, flat, h->pipe);
 }
 
 int scale_hip_set_terrain(scale_hip_ctx* h,

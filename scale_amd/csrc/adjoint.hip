@@ -45,25 +45,35 @@ struct Box {
   int k0, k1, i0, i1, j0, j1;
 };
 
-template <typename F>
+// The thread's index of a launch over n items: consecutive blocks of an XCD
+// are consecutive items (rows and levels that a stencil shares meet in one
+// L2), in 32 bits where n allows, as a division by a run-time extent costs
+// about 100 instructions in 64 bits, as much as a face's arithmetic, and 20
+// in 32.  The reverse sweep's face kernels at 128x128x64 take 3 to 10 % less.
+template <typename I>
+__device__ __forceinline__ I item() { return (I)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; }
+#define ITEMS_LAUNCH(n, tpb, K32, K64, ...)                                                                             \
+  do {                                                                                                                  \
+    const dim3 gr_((unsigned)(((n) + (tpb) - 1) / (tpb)));                                                              \
+    if ((n) < ((size_t)1 << 31)) hipLaunchKernelGGL(K32, gr_, dim3(tpb), 0, s, __VA_ARGS__);                            \
+    else hipLaunchKernelGGL(K64, gr_, dim3(tpb), 0, s, __VA_ARGS__);                                                    \
+    return hipGetLastError();                                                                                           \
+  } while (0)
+
+template <typename I, typename F>
 __global__ void __launch_bounds__(256) for3_kernel(Box b, F f) {
-  const int ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
-  const size_t n = (size_t)ni * (size_t)nj * (size_t)nk;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int i = b.i0 + (int)(t % (size_t)ni);
-  const size_t r = t / (size_t)ni;
-  const int j = b.j0 + (int)(r % (size_t)nj);
-  const int k = b.k0 + (int)(r / (size_t)nj);
-  f(k, i, j);
+  const I ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
+  const I t = item<I>();
+  if (t >= ni * nj * nk) return;
+  const I r = t / ni, q = r / nj;
+  f(b.k0 + (int)q, b.i0 + (int)(t - r * ni), b.j0 + (int)(r - q * nj));
 }
 
 template <typename F>
-hipError_t for3(Box b, F f, hipStream_t s) {
+hipError_t for3(Box b, F f, hipStream_t s, unsigned tpb = 256) {
   if (b.k1 < b.k0 || b.i1 < b.i0 || b.j1 < b.j0) return hipSuccess;
   const size_t n = (size_t)(b.i1 - b.i0 + 1) * (size_t)(b.j1 - b.j0 + 1) * (size_t)(b.k1 - b.k0 + 1);
-  hipLaunchKernelGGL(for3_kernel<F>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, f);
-  return hipGetLastError();
+  ITEMS_LAUNCH(n, tpb, (for3_kernel<unsigned, F>), (for3_kernel<size_t, F>), b, f);
 }
 
 #define HIPCHK(x)                          \
@@ -134,21 +144,19 @@ struct ZWin {
   double b[4] = {0.0, 0.0, 0.0, 0.0};
 };
 
-template <int DIR, typename F>
+template <typename I, int DIR, typename F>
 __global__ void __launch_bounds__(256) lseg_kernel(Dims d, Box b, int L, double* tgt, double* tgt2, F f) {
   const int ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
   // the fastest thread index and the other one across the lines (i and j,
   // i and k, j and k), and the line's own index (k, j, i)
   const int n1 = DIR == 2 ? nj : ni, n2 = DIR == 0 ? nj : nk, nl = DIR == 0 ? nk : (DIR == 1 ? nj : ni);
   const int nseg = (nl + L - 1) / L;
-  const size_t n = (size_t)n1 * (size_t)n2 * (size_t)nseg;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int c1 = (int)(t % (size_t)n1);
-  const size_t r = t / (size_t)n1;
-  const int c2 = (int)(r % (size_t)n2);
+  const I t = item<I>();
+  if (t >= (I)n1 * (I)n2 * (I)nseg) return;
+  const I r = t / (I)n1, sg = r / (I)n2;
+  const int c1 = (int)(t - r * (I)n1), c2 = (int)(r - sg * (I)n2);
   const int lb = DIR == 0 ? b.k0 : (DIR == 1 ? b.j0 : b.i0), le = DIR == 0 ? b.k1 : (DIR == 1 ? b.j1 : b.i1);
-  const int l0 = lb + (int)(r / (size_t)n2) * L, l1 = min(le, l0 + L - 1);
+  const int l0 = lb + (int)sg * L, l1 = min(le, l0 + L - 1);
   const int i = DIR == 2 ? 0 : b.i0 + c1;
   const int j = DIR == 2 ? b.j0 + c1 : (DIR == 0 ? b.j0 + c2 : 0);
   const int k = DIR == 0 ? 0 : b.k0 + c2;
@@ -192,20 +200,17 @@ struct XTgt {
   double* p[NT];
 };
 
-template <int NT, typename F>
+template <typename I, int NT, typename F>
 __global__ void __launch_bounds__(256) xrow_kernel(Dims d, Box b, XTgt<NT> tg, F f) {
-  const int ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
-  const size_t n = (size_t)ni * (size_t)nj * (size_t)nk;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const I ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
+  const I t = item<I>();
   XWin<NT> w;
 #pragma unroll
   for (int q = 0; q < NT; ++q) w.v[q][0] = w.v[q][1] = w.v[q][2] = w.v[q][3] = 0.0;
   long long p = -8;  // no point: never p-1 or p-2 of another lane's
-  if (t < n) {
-    const int i = b.i0 + (int)(t % (size_t)ni);
-    const size_t r = t / (size_t)ni;
-    const int j = b.j0 + (int)(r % (size_t)nj);
-    const int k = b.k0 + (int)(r / (size_t)nj);
+  if (t < ni * nj * nk) {
+    const I r = t / ni, q = r / nj;
+    const int i = b.i0 + (int)(t - r * ni), j = b.j0 + (int)(r - q * nj), k = b.k0 + (int)q;
     p = (long long)IX(d, k, i, j);
     f(k, i, j, w);
   }
@@ -230,8 +235,7 @@ template <int NT, typename F>
 hipError_t xrow(const Dims& d, Box b, XTgt<NT> tg, F f, hipStream_t s) {
   if (b.k1 < b.k0 || b.i1 < b.i0 || b.j1 < b.j0) return hipSuccess;
   const size_t n = (size_t)(b.i1 - b.i0 + 1) * (size_t)(b.j1 - b.j0 + 1) * (size_t)(b.k1 - b.k0 + 1);
-  hipLaunchKernelGGL((xrow_kernel<NT, F>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, b, tg, f);
-  return hipGetLastError();
+  ITEMS_LAUNCH(n, 256, (xrow_kernel<unsigned, NT, F>), (xrow_kernel<size_t, NT, F>), d, b, tg, f);
 }
 
 // Points of a box along z or y (DIR 0, 1), L consecutive points of a column
@@ -242,19 +246,17 @@ hipError_t xrow(const Dims& d, Box b, XTgt<NT> tg, F f, hipStream_t s) {
 // an atomic (the shifted targets of other threads reach the same points),
 // except, with OWN0, target 0's points that no other thread reaches (every
 // face q-2..q+1 of point q the thread's own).
-template <int DIR, int NT, bool OWN0, typename F>
+template <typename I, int DIR, int NT, bool OWN0, typename F>
 __global__ void __launch_bounds__(256) lsegn_kernel(Dims d, Box b, int L, XTgt<NT> tg, F f) {
   const int ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
   const int n2 = DIR == 0 ? nj : nk, nl = DIR == 0 ? nk : nj;
   const int nseg = (nl + L - 1) / L;
-  const size_t n = (size_t)ni * (size_t)n2 * (size_t)nseg;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int i = b.i0 + (int)(t % (size_t)ni);
-  const size_t r = t / (size_t)ni;
-  const int c2 = (int)(r % (size_t)n2);
+  const I t = item<I>();
+  if (t >= (I)ni * (I)n2 * (I)nseg) return;
+  const I r = t / (I)ni, sg = r / (I)n2;
+  const int i = b.i0 + (int)(t - r * (I)ni), c2 = (int)(r - sg * (I)n2);
   const int lb = DIR == 0 ? b.k0 : b.j0, le = DIR == 0 ? b.k1 : b.j1;
-  const int l0 = lb + (int)(r / (size_t)n2) * L, l1 = min(le, l0 + L - 1);
+  const int l0 = lb + (int)sg * L, l1 = min(le, l0 + L - 1);
   const int j = DIR == 0 ? b.j0 + c2 : 0, k = DIR == 0 ? 0 : b.k0 + c2;
   XWin<NT> w;
 #pragma unroll
@@ -291,17 +293,14 @@ hipError_t lseg(const Dims& d, Box b, double* tgt, double* tgt2, F f, hipStream_
   const size_t ni = b.i1 - b.i0 + 1, nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
   const size_t nl = DIR == 0 ? nk : (DIR == 1 ? nj : ni);
   const size_t n = ni * nj * nk / nl * ((nl + ZSEG_L - 1) / ZSEG_L);
-  hipLaunchKernelGGL((lseg_kernel<DIR, F>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, b, ZSEG_L, tgt, tgt2, f);
-  return hipGetLastError();
+  ITEMS_LAUNCH(n, 256, (lseg_kernel<unsigned, DIR, F>), (lseg_kernel<size_t, DIR, F>), d, b, ZSEG_L, tgt, tgt2, f);
 }
 template <int DIR, int NT, bool OWN0, typename F>
 hipError_t lsegn(const Dims& d, Box b, XTgt<NT> tg, F f, hipStream_t s) {
   if (b.k1 < b.k0 || b.i1 < b.i0 || b.j1 < b.j0) return hipSuccess;
   const size_t nl = DIR == 0 ? b.k1 - b.k0 + 1 : b.j1 - b.j0 + 1, n2 = DIR == 0 ? b.j1 - b.j0 + 1 : b.k1 - b.k0 + 1;
   const size_t n = (size_t)(b.i1 - b.i0 + 1) * n2 * ((nl + ZSEG_L - 1) / ZSEG_L);
-  hipLaunchKernelGGL((lsegn_kernel<DIR, NT, OWN0, F>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, b, ZSEG_L, tg,
-                     f);
-  return hipGetLastError();
+  ITEMS_LAUNCH(n, 256, (lsegn_kernel<unsigned, DIR, NT, OWN0, F>), (lsegn_kernel<size_t, DIR, NT, OWN0, F>), d, b, ZSEG_L, tg, f);
 }
 template <typename F>
 hipError_t zseg(const Dims& d, Box b, double* tgt, F f, hipStream_t s) { return lseg<0>(d, b, tgt, nullptr, f, s); }
@@ -844,7 +843,9 @@ static hipError_t stage_adj_t(Ctx& c, const StageAdjIO& io, hipStream_t st) {
   //     (the bands F1(k-1), F2(k), F3(k+1) of level k all read PT(k); A(k)
   //     is carried from the level below.  With few columns this runs about
   //     one wave per CU, so the loads go in chunks of ZCH levels, the next
-  //     chunk's in flight during the current chunk's work)
+  //     chunk's in flight during the current chunk's work; blocks of one
+  //     wave, so that 128x128 columns reach every CU: 47 us against 56 in
+  //     blocks of four, and 51 with chunks of 16)
   HIPCHK(for3(Box{0, 0, IS, IE, JS, JE}, [=] __device__(int, int i, int j) {
     constexpr int ZCH = 8;
     const size_t c0 = IX(d, 0, i, j);
@@ -915,7 +916,7 @@ _Pragma("unroll")
 _Pragma("unroll")
       for (int c = 0; c < ZCH; ++c) { dv[c] = ndv[c]; cv[c] = ncv[c]; }
     }
-  }, st));
+  }, st, 64));
   // (c) per level: adjoints of the band coefficients (through PT and
   //     A = dt^2 J33G RCDZ RT2P J33G / GSQRT) and of the right-hand side
   //     C = MOMZ + dt (pg + Sw), level L gathering rows L-1, L and L+1

@@ -1862,24 +1862,38 @@ hipError_t hevi_stage_traced(const StageIO& io, double* PT, double* St, double* 
   return launch_any(a, false, false, s);
 }
 
+// Rows of the FP32 tiles.  A block of 8 rows fills a CU (234 registers, 100 KB
+// of LDS), so up to one such tile per CU the rest of the chip is idle; two
+// blocks of 4 rows fit a CU, and a level of one takes less: large steps of
+// 96x96x64 (24 tiles of 8 rows) 1.97 ms against 2.24, 128x128x64 (32) 2.08
+// against 2.40, 256x200x64 (100) 2.47 against 2.91, 320x320x64 (200) 3.28
+// against 3.38.  Beyond, the rows staged twice cost more: 512x384x96 (384)
+// 9.95 against 9.71.  (2 rows: 2.20 at 128x128x64, 12.8 at 512x384x96.)
+static bool fp32_rows4(const Ctx& c) {
+  const Dims& d = c.d;
+  return ((d.IE - d.IS + 1 + 63) / 64) * ((d.JE - d.JS + 1 + 7) / 8) <= c.ncu;
+}
+template <int TJ>
+static void launch_fp32(const HeviArgsT<float>& a, int scheme, bool cmb, hipStream_t s) {
+  const Dims& d = a.d;
+  const unsigned ni = (unsigned)((d.IE - d.IS + 1 + 63) / 64), nb = ni * (unsigned)((d.JE - d.JS + TJ) / TJ);
+  const dim3 gr(nb), bl(64, TJ);
+  if (scheme == UD3) {
+    if (cmb) hipLaunchKernelGGL((hevi_tile<UD3, false, TJ, float, true>), gr, bl, 0, s, a, ni, nb);
+    else hipLaunchKernelGGL((hevi_tile<UD3, false, TJ, float, false>), gr, bl, 0, s, a, ni, nb);
+  } else {
+    if (cmb) hipLaunchKernelGGL((hevi_tile<CD4, false, TJ, float, true>), gr, bl, 0, s, a, ni, nb);
+    else hipLaunchKernelGGL((hevi_tile<CD4, false, TJ, float, false>), gr, bl, 0, s, a, ni, nb);
+  }
+}
 hipError_t hevi_stage(const StageIOT<float>& io, hipStream_t s) {
   HeviArgsT<float> a;
   fill_args(a, io);
   const Ctx& c = *io.ctx;
   if (c.terrain || io.divdmp_coef != 0.0) return hipErrorNotSupported;
-  const Dims& d = c.d;
-  const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1;
-  constexpr int TJ = 8;
-  const unsigned ni = (imax + 63) / 64, nb = ni * ((jmax + TJ - 1) / TJ);
   prof_start(c, "hevi_stage", s);
-  const bool cmb = io.combine != 0;
-  if (c.scheme == UD3) {
-    if (cmb) hipLaunchKernelGGL((hevi_tile<UD3, false, TJ, float, true>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-    else hipLaunchKernelGGL((hevi_tile<UD3, false, TJ, float, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-  } else {
-    if (cmb) hipLaunchKernelGGL((hevi_tile<CD4, false, TJ, float, true>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-    else hipLaunchKernelGGL((hevi_tile<CD4, false, TJ, float, false>), dim3(nb), dim3(64, TJ), 0, s, a, ni, nb);
-  }
+  if (fp32_rows4(c)) launch_fp32<4>(a, c.scheme, io.combine != 0, s);
+  else launch_fp32<8>(a, c.scheme, io.combine != 0, s);
   prof_stop(c, s);
   return hipGetLastError();
 }

@@ -505,9 +505,9 @@ struct ShortBufs {
 };
 
 // the inputs and outputs of stage r of a short step of length dts
-// the fourth RK4 stage combines the stages into the state itself (flat
-// HEVI on the tile kernel: FP32 always, FP64 where the tiles fill the device
-// or the stage is one of an ensemble's batched launches)
+// the fourth RK4 stage combines the stages into the state itself (HEVI: FP32
+// and an ensemble's batched launches always, FP64 on the tile kernel and on
+// the split kernels, not on the march that takes what those do not fit)
 template <typename R>
 static bool fused_rk4(const Ctx& c, bool batched) {
   const Model& M = *c.model;

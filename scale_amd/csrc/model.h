@@ -76,7 +76,7 @@ struct Ensemble {
   };
   // halo tables: the filter's fields, the outputs of stages 1..3, the state
   Tab halo[5];
-  // point tables of the large step's preparation and of the flux sum after
+  // point tables of the large step's preparation and of the flux mean after
   // each short step, every member in one launch
   Tab begin, sum;
   // the tracers of every member in batched launches, where the members have

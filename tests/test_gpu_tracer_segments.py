@@ -54,3 +54,26 @@ def test_model_tracers(hip, terrain):  # noqa: F811
             got.append([ctx.model_get(hip.QTRC_BASE + n) for n in range(case.qtrc.shape[-1])])
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("scheme", [3, 5], ids=["UD3", "UD5"])
+def test_ensemble_tracers_without_fct(hip, scheme):  # noqa: F811
+    """An ensemble without FCT (every stage on the tiles, or per point with
+    UD5): each member's tracers bit-identical to its own model's."""
+    print(f"[tracer segments] ensemble without FCT, scheme {scheme}", flush=True)
+    cases = [inputs.make_case(kmax=k, imax=i, jmax=j, noise=0.01, ntracer=2, tracer_kind=["blob", "tophat"], fct=False,
+                              momz_noise=0.05, v0=-2.0, scheme_tracer=scheme, halo=3 if scheme == 5 else 2)
+             for k, i, j in ((9, 12, 10), (14, 67, 6))]
+    alone = [hip.model_from_case(c) for c in cases]
+    members = [hip.model_from_case(c) for c in cases]
+    try:
+        with hip.Ensemble(members) as ens:
+            ens.large_step(2)
+            ens.synchronize()
+            for x, y in zip(alone, members):
+                x.model_large_step(2)
+                for n in range(2):
+                    assert np.array_equal(x.model_get(hip.QTRC_BASE + n), y.model_get(hip.QTRC_BASE + n))
+    finally:
+        for ctx in alone + members:
+            ctx.close()

@@ -508,7 +508,7 @@ static void fluxX_XVZ(const orc_grid *g, int s, double *flux, const double *mom,
 void orc_solve_direct(const orc_grid *g, double *C, const double *F1v, const double *F2v, const double *F3v) {
   GRID_LOCALS;
   const int KMAX = KE - KS + 1;
-  double e[512], f[512]; /* e(1..KMAX-2) at e[1..]; KA <= 512 is checked by the callers */
+  double e[ORC_KA_MAX], f[ORC_KA_MAX]; /* e(1..KMAX-2) at e[1..]; KA <= ORC_KA_MAX is checked by the stage */
   double *Cf = C - 1; /* Fortran C(1..KMAX-1) */
   double rdenom = 1.0 / F2v[KS];
   e[1] = -F1v[KS] * rdenom;
@@ -533,7 +533,7 @@ int orc_tstep_short_hevi(const orc_grid *g, int s,
     const double *num_diff, const double *wdamp_coef, double divdmp_coef, const double *DDIV,
     const orc_metric *m, const double *REF_dens, const double *REF_rhot, double dtrk) {
   GRID_LOCALS;
-  if (s != ORC_UD3 && s != ORC_CD4) return -1;
+  if ((s != ORC_UD3 && s != ORC_CD4) || KA > ORC_KA_MAX) return -1;
   const double *CDZ = m->CDZ, *FDZ = m->FDZ, *FDX = m->FDX, *FDY = m->FDY;
   const double *RCDZ = m->RCDZ, *RCDX = m->RCDX, *RCDY = m->RCDY;
   const double *RFDZ = m->RFDZ, *RFDX = m->RFDX, *RFDY = m->RFDY;
@@ -664,8 +664,8 @@ int orc_tstep_short_hevi(const orc_grid *g, int s,
 #pragma omp parallel for collapse(2) num_threads(g_threads) schedule(static)
   for (int j = JJS; j <= JJE; ++j)
     for (int i = IIS; i <= IIE; ++i) {
-      double A[512], F1v[512], F2v[512], F3v[512], PT[512], C[512];
-      double Mcol[512], Pcol[512];
+      double A[ORC_KA_MAX], F1v[ORC_KA_MAX], F2v[ORC_KA_MAX], F3v[ORC_KA_MAX], PT[ORC_KA_MAX], C[ORC_KA_MAX];
+      double Mcol[ORC_KA_MAX], Pcol[ORC_KA_MAX];
       for (int k = 0; k < KA; ++k) { Mcol[k] = MOMZ[I3(k, i, j)]; Pcol[k] = POTT[I3(k, i, j)]; }
       flux_valueW_Z(g, s, PT, Mcol, Pcol);
       for (int k = KS; k <= KE; ++k)

@@ -41,6 +41,8 @@ extern "C" {
 #define ORC_CD4 4
 #define ORC_UD5 5 /* tracer scheme: fifth-order upwind (ud5.F90), needs IHALO = JHALO = 3 */
 #define ORC_CD6 6 /* tracer scheme: sixth-order central (cd6.F90), needs IHALO = JHALO = 3 */
+/* levels (KA) of the column work arrays of the HEVI stage, which refuses more */
+#define ORC_KA_MAX 4104
 #define ORC_UD3KOREN 31 /* UD3KOREN1993: tracer scheme, UD3 with the Koren limiter */
 
 typedef struct {

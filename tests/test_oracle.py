@@ -146,8 +146,9 @@ def test_boundary_faces():
 
 
 # ---------------------------------------------------------------------------
-def test_thomas_matches_numpy_solve():
-    case = H.small_case(kmax=30, imax=4, jmax=4)
+@pytest.mark.parametrize("kmax", [30, 512, 1500])
+def test_thomas_matches_numpy_solve(kmax):
+    case = H.small_case(kmax=kmax, imax=4, jmax=4, dz=min(250.0, 20000.0 / kmax))
     g = case.grid
     rng = np.random.default_rng(0)
     n = g.KE - g.KS  # KMAX-1 unknowns
@@ -165,6 +166,19 @@ def test_thomas_matches_numpy_solve():
     rhs = rng.normal(size=n)
     x = po.solve_direct(g, rhs, F1, F2, F3)
     assert np.allclose(x, np.linalg.solve(A, rhs), rtol=1e-13, atol=1e-14)
+
+
+def test_stage_takes_deep_columns_and_refuses_deeper():
+    """A stage of 700 levels is finite everywhere; more levels than a column's
+    work arrays hold are refused."""
+    case = H.small_case(kmax=700, imax=4, jmax=3, dz=25.0)
+    g = case.grid
+    out = po.tstep_short_hevi(case, H.stage_inputs(case, seed=2, tend=False), 0.5)
+    for k in ("DENS_RK", "MOMZ_RK", "RHOT_RK"):
+        assert np.isfinite(out[k][g.KS:g.KE, g.IS:g.IE + 1, g.JS:g.JE + 1]).all(), k
+    deep = H.small_case(kmax=4101, imax=2, jmax=2, dz=5.0)
+    with pytest.raises(RuntimeError):
+        po.tstep_short_hevi(deep, H.stage_inputs(deep, seed=2), 0.5)
 
 
 # ---------------------------------------------------------------------------

@@ -867,6 +867,28 @@ __global__ void __launch_bounds__(1024) hevi_columns(HeviArgs a, unsigned ni, un
   }
 }
 
+// Columns per block of hevi_columns: the most, up to 32, that bound a block's
+// threads and LDS and give every CU a block; above 64 levels 16, so that two
+// blocks fit a CU.
+constexpr int columns_per_block(int imax, int jmax, int kmax, int ncu) {
+  const int ny = (kmax + SOLVE_L - 1) / SOLVE_L;
+  int cols = 32;
+  while (cols > 8 && ((cols > 16 && kmax > 64) || cols * ny > 1024 || (kmax - 1) * cols * 32 > SOLVE_LDS ||
+                      ((imax + cols - 1) / cols) * jmax < ncu))
+    cols /= 2;
+  return cols;
+}
+// every depth that hevi_split_fits takes, on grids of many columns and of few
+constexpr bool column_blocks_fit() {
+  for (int kmax = 4; kmax <= SOLVE_KMAX; ++kmax)
+    for (int n = 2; n <= 4096; n *= 2) {
+      const int cols = columns_per_block(n, n, kmax, 256);
+      if (cols * ((kmax + SOLVE_L - 1) / SOLVE_L) > 1024 || (kmax - 1) * cols * 32 > SOLVE_LDS) return false;
+    }
+  return true;
+}
+static_assert(column_blocks_fit(), "a block of hevi_columns exceeds its threads or LDS");
+
 // the tridiagonal rows of 8 columns fit in LDS, a field's byte offsets in 32 bits
 bool hevi_split_fits(const Dims& d) { return d.KE - d.KS + 1 <= SOLVE_KMAX && d.n3 < TILE_MAX_N3; }
 
@@ -901,9 +923,7 @@ static hipError_t launch(const HeviArgs& a, hipStream_t s) {
   const int imax = d.IE - d.IS + 1, jmax = d.JE - d.JS + 1, kmax = d.KE - d.KS + 1;
   if (2 * etiles(imax, jmax, 64) >= a.ctx->ncu) launch_etile<S, TERRAIN, DIVDMP, CMB, 64>(a, s);
   else launch_etile<S, TERRAIN, DIVDMP, CMB, 32>(a, s);
-  const int ny = (kmax + SOLVE_L - 1) / SOLVE_L;
-  int cols = 32;
-  while (cols > 8 && ((cols > 16 && kmax > 64) || (kmax - 1) * cols * 32 > SOLVE_LDS || ((imax + cols - 1) / cols) * jmax < a.ctx->ncu)) cols /= 2;
+  const int ny = (kmax + SOLVE_L - 1) / SOLVE_L, cols = columns_per_block(imax, jmax, kmax, a.ctx->ncu);
   const unsigned ni = (unsigned)((imax + cols - 1) / cols), nb = ni * (unsigned)jmax;
   const unsigned lds = (unsigned)((kmax - 1) * cols * 32);
   const dim3 b((unsigned)(cols * ny));

@@ -618,7 +618,7 @@ __global__ void __launch_bounds__(256) hevi_march(HeviArgs a, unsigned ni_tiles,
 
 // The split stage (hevi_split.hip) runs the general-metrics stage and the flat
 // grids the tile kernel does not take; SCALE_HIP_TERRAIN_SEG=0 and grids it
-// does not fit (more than 512 levels) keep the single-launch march.
+// does not fit (more than 4096 levels) keep the single-launch march.
 static bool split_enabled(const Ctx& c) {
   const char* e = getenv("SCALE_HIP_TERRAIN_SEG");
   return !(e && *e && atoi(e) <= 0) && hevi_split_fits(c.d);

@@ -722,7 +722,7 @@ __global__ void __launch_bounds__(TI * TJ, 2) hevi_etile(HeviArgs a, unsigned ni
 // against 159 at 128x128x64, 388 against 489 at 320x320x96.)
 constexpr int SOLVE_L = 4;          // levels per thread
 constexpr int SOLVE_LDS = 131072;   // bytes of LDS a block may take: 32 B per row and column
-constexpr int SOLVE_KMAX = SOLVE_LDS / (32 * 8);  // levels at 8 columns a block
+constexpr int SOLVE_KMAX = 1024 * SOLVE_L;  // levels at one column a block
 
 template <bool TERRAIN, bool CMB, int COLS>
 __global__ void __launch_bounds__(1024) hevi_columns(HeviArgs a, unsigned ni, unsigned nblocks) {
@@ -868,20 +868,23 @@ __global__ void __launch_bounds__(1024) hevi_columns(HeviArgs a, unsigned ni, un
 }
 
 // Columns per block of hevi_columns: the most, up to 32, that bound a block's
-// threads and LDS and give every CU a block; above 64 levels 16, so that two
-// blocks fit a CU.
+// threads and LDS, above 64 levels up to 16, so that two blocks fit a CU, and
+// down to 8 to give every CU a block.  More than 512 levels leave room for
+// fewer, whose loads fill less of a cache line: short step over terrain at
+// 64x64x600 4.9 ms and 64x64x1024 8.4 (4 columns), against 110 and 188 in the
+// one-launch march (hevi_march).
 constexpr int columns_per_block(int imax, int jmax, int kmax, int ncu) {
   const int ny = (kmax + SOLVE_L - 1) / SOLVE_L;
   int cols = 32;
-  while (cols > 8 && ((cols > 16 && kmax > 64) || cols * ny > 1024 || (kmax - 1) * cols * 32 > SOLVE_LDS ||
-                      ((imax + cols - 1) / cols) * jmax < ncu))
+  while (cols > 1 && (cols * ny > 1024 || (kmax - 1) * cols * 32 > SOLVE_LDS || (cols > 16 && kmax > 64) ||
+                      (cols > 8 && ((imax + cols - 1) / cols) * jmax < ncu)))
     cols /= 2;
   return cols;
 }
 // every depth that hevi_split_fits takes, on grids of many columns and of few
 constexpr bool column_blocks_fit() {
   for (int kmax = 4; kmax <= SOLVE_KMAX; ++kmax)
-    for (int n = 2; n <= 4096; n *= 2) {
+    for (int n = 2; n <= 4096; n *= 16) {
       const int cols = columns_per_block(n, n, kmax, 256);
       if (cols * ((kmax + SOLVE_L - 1) / SOLVE_L) > 1024 || (kmax - 1) * cols * 32 > SOLVE_LDS) return false;
     }
@@ -889,7 +892,7 @@ constexpr bool column_blocks_fit() {
 }
 static_assert(column_blocks_fit(), "a block of hevi_columns exceeds its threads or LDS");
 
-// the tridiagonal rows of 8 columns fit in LDS, a field's byte offsets in 32 bits
+// one column's tridiagonal rows fit a block, a field's byte offsets 32 bits
 bool hevi_split_fits(const Dims& d) { return d.KE - d.KS + 1 <= SOLVE_KMAX && d.n3 < TILE_MAX_N3; }
 
 // Tiles of TI x 8 columns.  64 columns re-read the smaller halo (1.59 cells per
@@ -927,9 +930,14 @@ static hipError_t launch(const HeviArgs& a, hipStream_t s) {
   const unsigned ni = (unsigned)((imax + cols - 1) / cols), nb = ni * (unsigned)jmax;
   const unsigned lds = (unsigned)((kmax - 1) * cols * 32);
   const dim3 b((unsigned)(cols * ny));
-  if (cols == 32) hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 32>), dim3(nb), b, lds, s, a, ni, nb);
-  else if (cols == 16) hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 16>), dim3(nb), b, lds, s, a, ni, nb);
-  else hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 8>), dim3(nb), b, lds, s, a, ni, nb);
+  switch (cols) {
+    case 32: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 32>), dim3(nb), b, lds, s, a, ni, nb); break;
+    case 16: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 16>), dim3(nb), b, lds, s, a, ni, nb); break;
+    case 8: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 8>), dim3(nb), b, lds, s, a, ni, nb); break;
+    case 4: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 4>), dim3(nb), b, lds, s, a, ni, nb); break;
+    case 2: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 2>), dim3(nb), b, lds, s, a, ni, nb); break;
+    default: hipLaunchKernelGGL((hevi_columns<TERRAIN, CMB, 1>), dim3(nb), b, lds, s, a, ni, nb);
+  }
   return hipGetLastError();
 }
 

@@ -15,9 +15,11 @@ pytestmark = pytest.mark.gpu
 # (kmax, imax, jmax): the fewest levels and columns; one column past a 32-column tile; one row past a tile; the
 # column blocks of hevi_columns: 260 rows of 9 to 18 columns take the widest block that fits (32 columns up to 64
 # levels, 16 up to 256, 8 beyond, with 102, 131, 66 and 66 KB of LDS at 200, 256, 257 and 258 levels), grids of few
-# columns 8 a block at any depth (512 levels: 131 KB); 129 tiles of 64 columns (the wide tile)
-SIZES = [(4, 2, 2), (5, 33, 9), (9, 31, 17), (6, 33, 130), (64, 18, 260), (65, 18, 130), (129, 9, 4), (200, 17, 130), (256, 17, 130),
-         (257, 6, 3), (257, 17, 130), (258, 17, 130), (512, 7, 5), (5, 65, 520)]
+# columns 8 a block up to 512 levels, any grid 4 up to 1024, 2 up to 2048, 1 up to 4096 and the one-launch march
+# beyond; 129 tiles of 64 columns (the wide tile)
+SIZES = [(4, 2, 2), (5, 33, 9), (9, 31, 17), (6, 33, 130), (64, 18, 260), (65, 18, 130), (129, 9, 4), (200, 17, 130),
+         (256, 17, 130), (257, 6, 3), (257, 17, 130), (258, 17, 130), (512, 7, 5), (513, 7, 5), (1024, 5, 3), (1025, 3, 5),
+         (2049, 3, 2), (4096, 2, 3), (4097, 2, 2), (5, 65, 520)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
@@ -26,7 +28,7 @@ SIZES = [(4, 2, 2), (5, 33, 9), (9, 31, 17), (6, 33, 130), (64, 18, 260), (65, 1
 def test_stage_sizes(hip, size, terrain, scheme, monkeypatch):  # noqa: F811
     monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", "1")
     print(f"[split stage] {size} terrain={terrain} scheme={scheme}", flush=True)
-    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=31, dz=80.0 if size[0] < 300 else 30.0)
+    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=31, dz=min(80.0, 15000.0 / size[0]))
     inp = H.stage_inputs(case, seed=29, coriolis=True)
     inp["wdamp_coef"] = np.linspace(0.0, 0.01, case.grid.KA)
     inp["divdmp_coef"] = 0.1 if size[2] % 2 else 0.0

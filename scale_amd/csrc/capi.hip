@@ -1164,7 +1164,8 @@ int scale_hip_model_set(scale_hip_ctx* h, int32_t f, const double* host) {
   const size_t n3 = c.d.n3;
   if (f == SCALE_HIP_CORIOLI) {
     if (int r = upload_raw(c, M->CORIOLI, host, c.d.pl)) return r;
-    M->has_coriolis = !all_equal(host, c.d.pl, 0.0);
+    const int cor = !all_equal(host, c.d.pl, 0.0);
+    if (cor != M->has_coriolis) { M->has_coriolis = cor; ++M->settings; }
     CK(hipStreamSynchronize(c.stream));
     return 0;
   }
@@ -1182,6 +1183,7 @@ int scale_hip_model_set(scale_hip_ctx* h, int32_t f, const double* host) {
     if (!M->RHOQ_tp) {
       M->RHOQ_tp = dalloc(c, n3 * (size_t)M->QA, &M->allocs);
       if (!M->RHOQ_tp) return fail("hipMalloc failed");
+      ++M->settings;
       CK(hipMemsetAsync(M->RHOQ_tp, 0, n3 * (size_t)M->QA * sizeof(double), c.stream));
     }
     return upload3(c, M->RHOQ_tp + n3 * (size_t)(f - SCALE_HIP_RHOQ_TP), host, 1);
@@ -1650,8 +1652,7 @@ int scale_hip_ensemble_set_graph(scale_hip_ensemble* h, int32_t on) {
   if (int r = check_ens(h)) return r;
   shp::Ensemble& E = h->E;
   CK(hipStreamSynchronize(E.stream));
-  if (E.exec) { (void)hipGraphExecDestroy(E.exec); E.exec = nullptr; }
-  if (E.graph) { (void)hipGraphDestroy(E.graph); E.graph = nullptr; }
+  shp::ensemble_drop_graph(E);
   E.use_graph = on != 0;
   return 0;
 }
@@ -1660,8 +1661,7 @@ static int ens_set_shape(shp::Ensemble& E, int stage_bpc, int nf_bpc, int nf_tj)
   if (stage_bpc < 0 || stage_bpc > 2 || nf_bpc < 0 || nf_bpc > 4 || (nf_tj != 4 && nf_tj != 8))
     return fail("ensemble shape: stage_bpc 0..2, nf_bpc 0..4 and nf_tj 4 or 8");
   CK(hipStreamSynchronize(E.stream));
-  if (E.exec) { (void)hipGraphExecDestroy(E.exec); E.exec = nullptr; }
-  if (E.graph) { (void)hipGraphDestroy(E.graph); E.graph = nullptr; }
+  shp::ensemble_drop_graph(E);
   const bool rebuild = nf_tj != E.nf_tj;
   E.stage_bpc = stage_bpc; E.nf_bpc = nf_bpc; E.nf_tj = nf_tj;
   if (rebuild) CK(shp::ensemble_build(E));

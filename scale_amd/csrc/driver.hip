@@ -1187,8 +1187,11 @@ hipError_t ensemble_build(Ensemble& E) {
   HIPCHK(ensemble_check(E, &why));
   E.built = false;
   hipError_t e = E.members[0]->model->mixed ? ensemble_build_t<float>(E) : ensemble_build_t<double>(E);
-  if (e == hipSuccess) E.built = true;
-  return e;
+  if (e != hipSuccess) return e;
+  E.settings.clear();
+  for (Ctx* cp : E.members) E.settings.push_back(cp->model->settings);
+  E.built = true;
+  return hipSuccess;
 }
 
 // one large step of every member in the phase-major order: the batched
@@ -1304,7 +1307,13 @@ static hipError_t ensemble_step_direct(Ensemble& E) {
 }
 
 hipError_t ensemble_large_step(Ensemble& E, int n) {
-  if (!E.built) HIPCHK(ensemble_build(E));
+  std::vector<unsigned> settings;
+  for (Ctx* cp : E.members) settings.push_back(cp->model->settings);
+  if (!E.built || settings != E.settings) {  // the steps in flight read the tables
+    HIPCHK(hipStreamSynchronize(E.stream));
+    ensemble_drop_graph(E);
+    HIPCHK(ensemble_build(E));
+  }
   // the members' pending work on their own streams comes first
   for (Ctx* cp : E.members) HIPCHK(hipStreamSynchronize(cp->stream));
   MemberStreams guard(E);
@@ -1329,6 +1338,12 @@ hipError_t ensemble_large_step(Ensemble& E, int n) {
   return E.members[0]->model->mixed ? ensemble_finish(E, n > 0) : hipSuccess;
 }
 
+void ensemble_drop_graph(Ensemble& E) {
+  if (E.exec) (void)hipGraphExecDestroy(E.exec);
+  if (E.graph) (void)hipGraphDestroy(E.graph);
+  E.exec = nullptr; E.graph = nullptr;
+}
+
 void ensemble_free(Ensemble& E) {
   if (E.stream) (void)hipStreamSynchronize(E.stream);
   for (int l = 0; l < Ensemble::MAX_LANES; ++l) {
@@ -1336,9 +1351,7 @@ void ensemble_free(Ensemble& E) {
     if (E.ev_lane[l]) { (void)hipEventDestroy(E.ev_lane[l]); E.ev_lane[l] = nullptr; }
   }
   if (E.ev_main) { (void)hipEventDestroy(E.ev_main); E.ev_main = nullptr; }
-  if (E.exec) (void)hipGraphExecDestroy(E.exec);
-  if (E.graph) (void)hipGraphDestroy(E.graph);
-  E.exec = nullptr; E.graph = nullptr;
+  ensemble_drop_graph(E);
   for (auto& b : E.stage) batch_free(b);
   batch_free(E.nf);
   for (auto& t : E.halo) tab_free(t);

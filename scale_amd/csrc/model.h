@@ -17,6 +17,9 @@ struct Model {
   double* CORIOLI = nullptr; // (IA,JA)
   double* wdamp_coef = nullptr;
   int has_coriolis = 0;
+  // changes of the settings that an ensemble's argument tables hold: RHOQ_tp
+  // given for the first time, has_coriolis
+  unsigned settings = 0;
   // outputs of the last large step
   double *mflx_hi = nullptr, *tflx_hi = nullptr;
   // large-step work arrays
@@ -90,7 +93,9 @@ struct Ensemble {
   std::vector<BatchBuf> tr_s1, tr_s2, tr_ph, tr_s3;
   Tab tr_mf, tr_q1, tr_q2, tr_r;
   std::vector<Tab> tr_q, tr_copy;
+  // the tables are built, at these settings of the members
   bool built = false;
+  std::vector<unsigned> settings;
   // lanes: streams the members' own launches spread over (member m on lane
   // m % nlanes), forked from and joined back to `stream` around each batched
   // launch, so that the small per-member kernels of different members overlap
@@ -106,6 +111,7 @@ struct Ensemble {
 hipError_t ensemble_check(const Ensemble& E, const char** why);
 hipError_t ensemble_build(Ensemble& E);
 hipError_t ensemble_large_step(Ensemble& E, int n);
+void ensemble_drop_graph(Ensemble& E);
 void ensemble_free(Ensemble& E);
 
 // rec (FP64 flat HEVI without divergence damping, one short step per large

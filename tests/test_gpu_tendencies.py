@@ -1,4 +1,6 @@
-"""Tendencies given to a model after steps without any, against the oracle."""
+"""Tendencies given to a model after steps without any, against the oracle, and
+settings given to the members of an ensemble after its creation, against the
+members' own models."""
 import numpy as np
 import pytest
 
@@ -69,6 +71,45 @@ def test_tendencies_given_to_a_replayed_ensemble(hip, mixed, nstep):  # noqa: F8
                 ens.synchronize()
                 for case, x, y in zip(cases, alone, members):
                     for f in hip.STATE + ("mflx_hi",) + tuple(hip.QTRC_BASE + n for n in range(case.qtrc.shape[-1])):
+                        assert np.array_equal(x.model_get(f), y.model_get(f)), (given, f)
+    finally:
+        for ctx in alone + members:
+            ctx.close()
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["direct", "replayed"])
+@pytest.mark.parametrize("fct", [False, True], ids=["plain", "fct"])
+@pytest.mark.parametrize("scheme", [3, 6], ids=["UD3", "CD6"])
+def test_settings_given_to_an_ensemble(hip, graph, fct, scheme):  # noqa: F811
+    """Members are given a tracer tendency (UD3: tracers in batched launches, CD6: on their own) and the Coriolis
+    parameter after steps without, and the parameter's zeros again after that: each stays bit-identical to its own
+    model."""
+    kw = dict(scheme_tracer=scheme, fct=fct, halo=3 if scheme == 6 else 2)
+    cases = [H.small_case(kmax=10, imax=9, jmax=6, seed=46, **kw), H.small_case(kmax=12, imax=66, jmax=5, seed=47, **kw)]
+    rng = np.random.Generator(np.random.PCG64(10))
+    tps = []
+    for case in cases:
+        g = case.grid
+        a = g.zeros()
+        a[:, g.IS:g.IE + 1, g.JS:g.JE + 1] = 1e-3 * rng.standard_normal((g.KA, g.imax, g.jmax))
+        tps.append(inputs.halo_fill(g, a))
+    alone = [hip.model_from_case(c) for c in cases]
+    members = [hip.model_from_case(c) for c in cases]
+    try:
+        with hip.Ensemble(members) as ens:
+            ens.set_graph(graph)
+            for given in ("nothing", "RHOQ_tp", "CORIOLI", "zeros"):
+                for case, ctx, tp in zip(cases + cases, alone + members, tps + tps):
+                    if given == "RHOQ_tp":
+                        ctx.model_set(hip.RHOQ_TP_BASE + 1, tp)
+                    elif given != "nothing":
+                        ctx.model_set("CORIOLI", np.full(case.corioli.shape, 1e-2 if given == "CORIOLI" else 0.0, order="F"))
+                for ctx in alone:
+                    ctx.model_large_step(2)
+                ens.large_step(2)
+                ens.synchronize()
+                for case, x, y in zip(cases, alone, members):
+                    for f in hip.STATE + tuple(hip.QTRC_BASE + n for n in range(case.qtrc.shape[-1])):
                         assert np.array_equal(x.model_get(f), y.model_get(f)), (given, f)
     finally:
         for ctx in alone + members:

@@ -1,6 +1,6 @@
 """The drop-in stage's transfers through pinned slots (calls of 32 MB and more:
 partial last chunks, arrays of several chunks and of one) and its look at the
-metrics, bit for bit against the oracle."""
+metrics (terrain seen before the uploads and after them), bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -10,8 +10,9 @@ from test_gpu_parity import OUTS, hip, oracle_stage, run_stage_gpu  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-# (kmax, imax, jmax): arrays of 0.9 MB, num_diff of four chunks; of 4.1 MB, two chunks
-@pytest.mark.parametrize("size", [(40, 47, 48), (60, 91, 85)], ids=lambda s: "x".join(map(str, s)))
+# (kmax, imax, jmax): a call below 32 MB, array by array; arrays of 0.9 MB, num_diff of four chunks; of 4.1 MB, two
+# chunks, and more columns than the first look at the metrics takes
+@pytest.mark.parametrize("size", [(9, 12, 10), (40, 47, 48), (60, 91, 85)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("metric", ["flat", "terrain", "one element"])
 def test_stage_transfers(hip, size, metric):  # noqa: F811
     print(f"[drop-in] {size} {metric}", flush=True)

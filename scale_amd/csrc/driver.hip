@@ -1041,11 +1041,16 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
   const int n = (int)E.members.size();
   std::vector<const Ctx*> cs;
   for (Ctx* cp : E.members) cs.push_back(cp);
-  // every stage on LDS tiles for the two-cell schemes (the tiles of all
-  // members keep every CU busy even where one member's would not)
+  // the FCT stage on LDS tiles for the two-cell schemes.  The stages without
+  // FCT follow from two tiles per CU on; with fewer the tiles' march up whole
+  // columns takes longer than the points' repeated loads.
+  // Large steps with three tracers, no FCT, points | tiles: 40x40x80 (10 tiles)
+  // 4.09 | 4.94 ms, 6 of 64x64x40 and 96x40x30 (108) 2.90 | 3.24, 6 of
+  // 128x128x64 (384) 6.63 | 6.78, 8 (512) 7.59 | 7.46, 64 (4096) 58.8 | 55.9
   const int st = E.members[0]->scheme_tracer;
   E.tr_tile = (st == UD3 || st == CD4 || st == UD3KOREN || st == UD1 || st == CD2);
   for (const Ctx* cp : cs) E.tr_tile = E.tr_tile && cp->d.n3 < TILE_MAX_N3;
+  E.tr_plain = E.tr_tile && trt_batch_tiles(cs.data(), n) >= 2u * (unsigned)E.ncu;
   for (auto* v : {&E.tr_s1, &E.tr_s2, &E.tr_ph, &E.tr_s3})
     for (auto& b : *v) batch_free(b);
   for (auto* v : {&E.tr_q, &E.tr_copy})
@@ -1076,13 +1081,16 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
       cp_blocks.push_back((unsigned)((nn + 1023) / 1024));
       qf.push_back({cp, q});
     }
-    if (E.tr_tile) {
-      HIPCHK(trt_batch_build(cs.data(), s1.data(), n, E.tr_s1[(size_t)iq]));
-      HIPCHK(trt_batch_build(cs.data(), s2.data(), n, E.tr_s2[(size_t)iq]));
+    auto plain = [&](const std::vector<TracerIO>& ios, BatchBuf& b) {
+      return E.tr_plain ? trt_batch_build(cs.data(), ios.data(), n, b) : tracer_batch_build(cs.data(), ios.data(), n, false, b);
+    };
+    HIPCHK(plain(s1, E.tr_s1[(size_t)iq]));
+    HIPCHK(plain(s2, E.tr_s2[(size_t)iq]));
+    if (!M0.fct) {
+      HIPCHK(plain(s3, E.tr_s3[(size_t)iq]));
+    } else if (E.tr_tile) {
       HIPCHK(trt_batch_build(cs.data(), s3.data(), n, E.tr_s3[(size_t)iq]));
     } else {
-      HIPCHK(tracer_batch_build(cs.data(), s1.data(), n, false, E.tr_s1[(size_t)iq]));
-      HIPCHK(tracer_batch_build(cs.data(), s2.data(), n, false, E.tr_s2[(size_t)iq]));
       HIPCHK(tracer_batch_build(cs.data(), s3.data(), n, true, E.tr_ph[(size_t)iq]));
       HIPCHK(tracer_batch_build(cs.data(), s3.data(), n, false, E.tr_s3[(size_t)iq]));
     }
@@ -1113,7 +1121,7 @@ static hipError_t ensemble_tracers_build(Ensemble& E) {
 static hipError_t ensemble_tracers(Ensemble& E, hipStream_t s) {
   HIPCHK(halo_table_launch<double>(E.tr_mf, s));
   for (int iq = 0; iq < E.tr_qa; ++iq) {
-    auto nofct = [&](const BatchBuf& b) { return E.tr_tile ? trt_batch_launch(b, 2, s) : tracer_batch_launch(b, 0, s); };
+    auto nofct = [&](const BatchBuf& b) { return E.tr_plain ? trt_batch_launch(b, 2, s) : tracer_batch_launch(b, 0, s); };
     HIPCHK(nofct(E.tr_s1[(size_t)iq]));  // stage 1: dt/3, no FCT
     HIPCHK(halo_table_launch<double>(E.tr_q1, s));
     HIPCHK(nofct(E.tr_s2[(size_t)iq]));  // stage 2: dt/2, no FCT

@@ -230,6 +230,7 @@ hipError_t tracer_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, 
 hipError_t tracer_batch_launch(const BatchBuf& b, int kind, hipStream_t s);
 // the same on LDS tiles (tracer_tile.hip; two-cell schemes): kinds 0 R+/R-
 // (phi_lo within), 1 the update, 2 the stage without FCT
+unsigned trt_batch_tiles(const Ctx* const* cs, int n);  // tiles of a launch
 hipError_t trt_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, BatchBuf& b);
 hipError_t trt_batch_launch(const BatchBuf& b, int kind, hipStream_t s);
 // ATMOS_DYN_numfilter_coef_q (ND_ORDER = 1) with the halo fill of its 3

@@ -559,6 +559,15 @@ hipError_t tracer_stage_tile(const Ctx& c, const TracerIO& io, double* rjpls, do
   }
 }
 
+static unsigned batch_tiles(const Dims& d) {
+  return (unsigned)((d.IE - d.IS + 1 + 63) / 64) * (unsigned)((d.JE - d.JS + 1 + TT_TJ - 1) / TT_TJ);
+}
+unsigned trt_batch_tiles(const Ctx* const* cs, int n) {
+  unsigned t = 0;
+  for (int m = 0; m < n; ++m) t += batch_tiles(cs[m]->d);
+  return t;
+}
+
 // the stages of every member on tiles (the members' stage arguments;
 // flat terrain, one two-cell scheme, one bound kind)
 hipError_t trt_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, BatchBuf& b) {
@@ -582,7 +591,7 @@ hipError_t trt_batch_build(const Ctx* const* cs, const TracerIO* ios, int n, Bat
     a.GSQRT = nullptr; a.MAPF = nullptr; a.dens_mode = io.dens_mode;
     const Dims& d = c.d;
     ni[(size_t)m] = (unsigned)((d.IE - d.IS + 1 + 63) / 64);
-    first[(size_t)m + 1] = first[(size_t)m] + ni[(size_t)m] * (unsigned)((d.JE - d.JS + 1 + TT_TJ - 1) / TT_TJ);
+    first[(size_t)m + 1] = first[(size_t)m] + batch_tiles(d);
   }
   const hipError_t e = batch_upload(args, first, ni, b);
   b.scheme = scheme; b.tj = along;

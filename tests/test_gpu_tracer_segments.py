@@ -56,14 +56,11 @@ def test_model_tracers(hip, terrain):  # noqa: F811
         assert np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("scheme", [3, 5], ids=["UD3", "UD5"])
-def test_ensemble_tracers_without_fct(hip, scheme):  # noqa: F811
-    """An ensemble without FCT (every stage on the tiles, or per point with
-    UD5): each member's tracers bit-identical to its own model's."""
-    print(f"[tracer segments] ensemble without FCT, scheme {scheme}", flush=True)
-    cases = [inputs.make_case(kmax=k, imax=i, jmax=j, noise=0.01, ntracer=2, tracer_kind=["blob", "tophat"], fct=False,
+def ensemble_tracers(hip, sizes, scheme, fct):  # noqa: F811
+    """Two large steps of an ensemble: each member's tracers bit-identical to its own model's."""
+    cases = [inputs.make_case(kmax=k, imax=i, jmax=j, noise=0.01, ntracer=2, tracer_kind=["blob", "tophat"], fct=fct,
                               momz_noise=0.05, v0=-2.0, scheme_tracer=scheme, halo=3 if scheme == 5 else 2)
-             for k, i, j in ((9, 12, 10), (14, 67, 6))]
+             for k, i, j in sizes]
     alone = [hip.model_from_case(c) for c in cases]
     members = [hip.model_from_case(c) for c in cases]
     try:
@@ -77,3 +74,19 @@ def test_ensemble_tracers_without_fct(hip, scheme):  # noqa: F811
     finally:
         for ctx in alone + members:
             ctx.close()
+
+
+@pytest.mark.parametrize("scheme", [3, 5], ids=["UD3", "UD5"])
+def test_ensemble_tracers_without_fct(hip, scheme):  # noqa: F811
+    """An ensemble of few columns without FCT: every stage per point."""
+    print(f"[tracer segments] ensemble without FCT, scheme {scheme}", flush=True)
+    ensemble_tracers(hip, ((9, 12, 10), (14, 67, 6)), scheme, False)
+
+
+@pytest.mark.parametrize("scheme", [3, 31], ids=["UD3", "Koren"])
+@pytest.mark.parametrize("fct", [False, True], ids=["plain", "fct"])
+def test_ensemble_tracers_on_tiles(hip, scheme, fct):  # noqa: F811
+    """An ensemble of two tiles of 64 x 4 columns per CU and more: the stages
+    without FCT on the tiles too."""
+    print(f"[tracer segments] ensemble on tiles, scheme {scheme}, fct={fct}", flush=True)
+    ensemble_tracers(hip, ((9, 12, 10), (6, 67, 1030)), scheme, fct)

@@ -1,7 +1,8 @@
 """The split FP64 stage (hevi_etile + hevi_columns) at the sizes where it can go
 wrong: tile, segment and column-block edges, remainders, the fewest levels, and
 level counts on both sides of every column-block width, bit for bit against the
-oracle; the RK4 combination fused into both kernels."""
+oracle; the RK4 combination fused into both kernels; the rule that chooses
+between them and the tile kernel on flat grids."""
 import numpy as np
 import pytest
 
@@ -42,21 +43,27 @@ def test_stage_sizes(hip, size, terrain, scheme, monkeypatch):  # noqa: F811
 
 @pytest.mark.parametrize("size", [(4, 2, 2), (9, 65, 9), (33, 30, 7), (70, 33, 6)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("terrain", [False, True], ids=["flat", "terrain"])
-def test_fused_combination(hip, size, terrain, monkeypatch):  # noqa: F811
-    """Three large steps through the combining fourth stage, within 1e-12 of
-    each field's scale (pow() in the preparation)."""
+@pytest.mark.parametrize("forced", [False, True], ids=["plain", "forced"])
+def test_fused_combination(hip, size, terrain, forced, monkeypatch):  # noqa: F811
+    """Three large steps through the combining fourth stage, without and with
+    divergence damping, Coriolis force and sponge layer, within 1e-12 of each
+    field's scale (pow() in the preparation)."""
     monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", "1")
-    print(f"[split stage] model {size} terrain={terrain}", flush=True)
+    print(f"[split stage] model {size} terrain={terrain} forced={forced}", flush=True)
     case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=37, dz=100.0)
+    divdmp = 0.2 if forced else 0.0
+    if forced:
+        case.corioli[:] = 1.0e-2
+        case.wdamp_coef[:] = np.linspace(0.0, 0.01, case.grid.KA)
     zs = inputs.bell_topography(case.grid, height=60.0, half_width=1500.0) if terrain else None
     ocase = case
     if terrain:
         ocase = inputs.Case(**{**case.__dict__, "metric": {**case.metric, **po.terrain_metrics(case.grid, zs, case.fz, case.metric)}})
-    m = po.Model(ocase)
+    m = po.Model(ocase, divdmp_coef=divdmp)
     m.step(3)
     g = case.grid
     sl = (slice(g.KS, g.KE + 1), slice(g.IS, g.IE + 1), slice(g.JS, g.JE + 1))
-    with hip.model_from_case(case, zsfc=zs) as ctx:
+    with hip.model_from_case(case, zsfc=zs, divdmp_coef=divdmp) as ctx:
         ctx.model_large_step(3)
         for k in hip.STATE:
             got, ref = ctx.model_get(k), m.state[k]
@@ -64,3 +71,24 @@ def test_fused_combination(hip, size, terrain, monkeypatch):  # noqa: F811
         for k in ("mflx_hi", "tflx_hi"):
             got, ref = ctx.model_get(k)[sl], getattr(m, k)[sl]
             assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max(), k
+
+
+@pytest.mark.parametrize("rows", [1840, 1848, 2049, 3680, 3688])
+def test_flat_route(hip, rows, monkeypatch):  # noqa: F811
+    """The rule between the tile kernel and the split launches left alone, on
+    256 CUs: 230 tiles of 64 x 8 columns | 231 (90 % of a round), 257 and 460 |
+    461 (90 % of two).  A stage bit for bit the oracle's, two large steps
+    within 1e-12 of each field's scale."""
+    monkeypatch.delenv("SCALE_HIP_FLAT_SPLIT")
+    print(f"[split stage] flat route, {rows} rows", flush=True)
+    case = H.small_case(kmax=5, imax=3, jmax=rows, seed=39, dz=100.0)
+    inp = H.stage_inputs(case, seed=29, coriolis=True)
+    ref, got = oracle_stage(case, inp, 0.5), run_stage_gpu(hip, case, inp, 0.5)
+    for k in OUTS:
+        H.compare(ref[k], got[k], k)
+    m = po.Model(case)
+    m.step(2)
+    with hip.model_from_case(case) as ctx:
+        ctx.model_large_step(2)
+        for k in hip.STATE:
+            assert np.abs(ctx.model_get(k) - m.state[k]).max() <= 1e-12 * max(np.abs(m.state[k]).max(), 1.0), k

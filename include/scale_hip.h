@@ -380,9 +380,10 @@ int scale_hip_batch_adjoint(scale_hip_ctx *const *members, int32_t n, double *co
  * order.
  *   SCALE_HIP_TUNE_NF_TJ: rows of the numerical-filter tile, 4, 8 or 16
  *   (0 = chosen from the grid).
- *   SCALE_HIP_TUNE_TRACER_TILE: the FCT tracer stage on LDS tiles (flat
- *   terrain; UD3, CD4, UD3KOREN1993, UD1 and CD2): 1 (default) where the grid
- *   gives every CU two tiles, 2 always, 0 never (per-point kernels).
+ *   SCALE_HIP_TUNE_TRACER_TILE: the tracer stages on LDS tiles (UD3, CD4,
+ *   UD3KOREN1993, UD1 and CD2, flat terrain or not): 1 (default) where the
+ *   tiles of 64 x 4 columns give every CU eight levels of one, 2 always,
+ *   0 never (per-point kernels).
  *   SCALE_HIP_TUNE_ADJ_TAPE: the number of trailing segments (of `every`
  *   steps) whose tapes (the step states and the 45 fields per step the
  *   reverse step reads, 400 B per grid point and step) the checkpointed

@@ -636,9 +636,9 @@ static hipError_t launch_march(const HeviArgs& a, hipStream_t s) {
 // The flat stage on the tile kernel, or split.  The tile kernel runs one block
 // a CU, so its time goes in rounds of ncu tiles: it takes grids whose tiles
 // fill at least 90 % of them.  RK4 short step, tile | split: 512x512x128 (two
-// full rounds) 20.5 | 21.5 ms, 512x512x64 10.2 | 10.3, 320x320x96 (0.78 of a
+// full rounds) 20.6 | 21.6 ms, 512x512x64 10.3 | 10.4, 320x320x96 (0.78 of a
 // round) 7.0 | 6.8, 448x320x96 (1.09) 13.3 | 9.5, 128x128x64 (0.13) 3.6 |
-// 0.76.  SCALE_HIP_FLAT_SPLIT=0 keeps the tile kernel, =1 the split launches,
+// 0.79.  SCALE_HIP_FLAT_SPLIT=0 keeps the tile kernel, =1 the split launches,
 // whatever the grid.
 bool hevi_flat_tile(const Ctx& c) {
   const char* e = getenv("SCALE_HIP_FLAT_SPLIT");

@@ -56,9 +56,9 @@ struct MetO {
 // a launch of its own.
 // Bound by memory latency at two waves per SIMD (its registers and LDS): at
 // 512x512x128 flat 2.72 ms, 317 B of HBM traffic a point (208 read and 80
-// written at least) at 3.9 TB/s; the next level's num_diff of the faces is
-// loaded ahead (22.7 -> 22.3 ms per short step there), the ring's level too
-// spills and is slower (26.1 ms).  One thread per point reading its stencil
+// written at least) at 3.9 TB/s.  The next level's num_diff of the faces is
+// loaded ahead (2 % of a short step there); the ring's level too spills and is
+// slower (by 17 %).  One thread per point reading its stencil
 // through the caches, a launch per section, was the kernel before: 215 us
 // against 105 for the flat explicit part at 128x128x64, 458 against 273 with
 // general metrics, 2.88 ms against 1.59 at 301x259x80.

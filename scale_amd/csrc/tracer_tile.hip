@@ -80,8 +80,8 @@ __device__ __forceinline__ double tt_hz(const Dims& d, int kk, double vel, const
 // of members
 //
 // Bound by FP64 instruction issue (the along-stream bounds are six divisions
-// and 112 multiply-adds of LDS operands) and its latency at three wavefronts
-// per SIMD.  A thread owns a cell: phi_lo, the faces and P+/P- of level u,
+// and 112 multiply-adds of LDS operands): at three wavefronts per SIMD each
+// issues for 30 % of its time.  A thread owns a cell: phi_lo, the faces and P+/P- of level u,
 // then, a barrier later, R+/R- of level u - 1, for which it keeps six values
 // in registers; the ring's cells are one item each of the first threads, and
 // every load of a level is issued before its first barrier.  Sharing the
@@ -318,9 +318,9 @@ __global__ void __launch_bounds__(64 * TJ, 3) trt_ratio(TtArgs a, unsigned ni_ti
 // shares them through LDS, but with one barrier a level (the tiles alternate
 // between two slots), no items beside the cells, and few enough registers
 // that three blocks of 4 wavefronts (LIM; two of 8 without) cover each
-// other's loads.  At 320x320x96: 0.216 ms (4 TB/s) against 0.331 with shared
+// other's loads.  At 320x320x96: 0.217 ms (4.5 TB/s) against 0.331 with shared
 // faces and the next level's loads in flight at one block per CU; 8 rows
-// 0.25-0.27; without FCT 0.157 (4 TB/s) against 0.172.
+// 0.25-0.27; without FCT 0.154 (4.5 TB/s) against 0.172.
 template <int S, int TJ, bool LIM, bool TER>
 __device__ __forceinline__ void trt_update_body(const TtArgs& a, unsigned lb, unsigned ni_tiles, int k0, int k1) {
   constexpr int W2 = 68, H2 = TJ + 4, W1 = 66, H1 = TJ + 2, NT = 64 * TJ;

@@ -41,7 +41,7 @@ def test_stage_sizes(hip, size, terrain, scheme, monkeypatch):  # noqa: F811
         H.compare(ref[k], got[k], k)
 
 
-@pytest.mark.parametrize("size", [(4, 2, 2), (9, 65, 9), (33, 30, 7), (70, 33, 6)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("size", [(4, 2, 2), (9, 65, 9), (33, 30, 7), (70, 33, 6), (520, 5, 3)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("terrain", [False, True], ids=["flat", "terrain"])
 @pytest.mark.parametrize("forced", [False, True], ids=["plain", "forced"])
 def test_fused_combination(hip, size, terrain, forced, monkeypatch):  # noqa: F811
@@ -50,7 +50,7 @@ def test_fused_combination(hip, size, terrain, forced, monkeypatch):  # noqa: F8
     field's scale (pow() in the preparation)."""
     monkeypatch.setenv("SCALE_HIP_FLAT_SPLIT", "1")
     print(f"[split stage] model {size} terrain={terrain} forced={forced}", flush=True)
-    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=37, dz=100.0)
+    case = H.small_case(kmax=size[0], imax=size[1], jmax=size[2], seed=37, dz=min(100.0, 15000.0 / size[0]))
     divdmp = 0.2 if forced else 0.0
     if forced:
         case.corioli[:] = 1.0e-2
